@@ -6,16 +6,20 @@
 // token-major with arbitrary token strides and head stride 64, so q, k and v
 // can be read straight out of the fused qkv projection output.
 //
-// Workgroup: ATT_WAVES waves, 64 queries each (64 * ATT_WAVES queries of one
-// (sequence, head)).
-// Per 64-key tile a wave computes S^T = K Q^T for its two 32-query blocks
-// (2 x 2 x 4 v_mfma_f32_32x32x16_f16, every K fragment read from LDS feeding
-// both blocks), the online softmax in registers, and O^T += V^T P^T (16 more
-// MFMAs, each V^T fragment again feeding both blocks).
+// Workgroup: 4 waves of QB 32-query blocks each (128 QB queries of one
+// (sequence, head); QB = 2 or 1, see attention_fwd_kernel).
+// Per 64-key tile a wave computes S^T = K Q^T for its query blocks
+// (QB x 2 x 4 v_mfma_f32_32x32x16_f16, every K fragment read from LDS feeding
+// all its blocks), the online softmax in registers, and O^T += V^T P^T (as
+// many MFMAs again, each V^T fragment likewise shared).
 // The softmax is trimmed to what the MFMAs cannot hide: key masking only on
 // the last (partial) tile; Q pre-scaled by scale * log2(e) and the score
 // accumulators started at -m (the running reference), so P = 2^S takes one
-// exp2 per score and nothing else; row sums by v_dot2 on the fp16 P values;
+// exp2 per score and nothing else; row sums by one fp32 add per score (a
+// v_dot2 of the packed fp16 pair is one instruction instead of two, but beside
+// MFMAs in flight it cost ~16 cycles: a 32 x 64 tile's 16 MFMAs, 32 exp2 and
+// packs took 527 cycles alone, 781 with 16 v_dot2, 541 with 32 adds; 43968
+// tokens 7.87 -> 7.74 ms, 10992 541 -> 526 us, same box);
 // and a lazy rescale -- the reference moves only when a tile exceeds it by
 // 2^8, so most tiles skip the O *= alpha pass, and the tile maximum itself is
 // only computed when a lane's tile sum says some P may have exceeded 2^8.
@@ -28,10 +32,10 @@
 //    registers 8p..8p+7 of block kb, i.e. keys 32kb + 16p + {0..3, 8..11} + 4h.
 //  * K and V tiles arrive by LDS DMA in their natural [key][dim] layout
 //    (128-byte rows; 16-byte chunk c of row r at c ^ fk(r) for K and
-//    c ^ fv(r) for V), one DMA tile ahead.  In the 4-wave form a DMA tile
-//    holds 128 keys, consumed as two 64-key compute tiles, so the workgroup
-//    meets at one barrier per 128 keys (1-2 % faster than one per 64,
-//    bit-identical); the 2-wave form copies 64-key tiles.
+//    c ^ fv(r) for V), one DMA tile ahead.  At QB = 2 a DMA tile holds 128
+//    keys, consumed as two 64-key compute tiles, so the workgroup meets at
+//    one barrier per 128 keys (1-2 % faster than one per 64, bit-identical);
+//    at QB = 1 it copies 64-key tiles.
 //  * V^T (the PV A operand) comes out of LDS through ds_read_b64_tr_b16: two
 //    transposed 8-byte reads give each lane its dim's 8 keys in k-slot order,
 //    with no register staging or transposed stores.
@@ -39,17 +43,7 @@
 
 namespace qv {
 
-constexpr int ATT_QW = 64;                 // queries per wave (two 32-query blocks)
 constexpr int ATT_BK = 64;                 // keys per compute tile
-// The kernel's two forms (template WAVES, SUB): 4 waves per workgroup with
-// 128-key DMA tiles (64 KB of K / V buffers, two workgroups per CU), and, for
-// launches that would not fill one round of those, 2 waves with 64-key DMA
-// tiles (32 KB, four workgroups per CU), which spreads the queries over twice
-// as many workgroups (bit-identical: the key order of every query is the
-// same; 4 x 1374 frame tokens 0.5-5 % and one 5496-token sequence 1.8 %
-// faster, two boxes).  At 8 x 1374 (1.5 rounds of the 4-wave form) the
-// 2-wave form was 7-8 % slower: twice the K / V copies per query and a
-// barrier per 64 keys.
 
 constexpr float RESCALE_SLACK = 8.0f;  // log2 units: P <= 256 between rescales
 constexpr float P_SUM_LIMIT = 256.0f;  // 2^RESCALE_SLACK: a lane's tile sum above it may hide a P above it
@@ -93,11 +87,26 @@ __device__ __forceinline__ float half_sum(float x) {
   return a + b;
 }
 
-template <int WAVES, int SUB>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_fwd_kernel(
+// Two forms, bit-identical (a query's keys come in the same order, and the
+// lazy rescale of a query depends on its own scores alone):
+//  * wide (QB = 2): 64 queries a wave, 256 VGPRs, two 64 KB workgroups a CU.
+//    Every LDS fragment feeds two MFMAs; bound by VALU issue and by what of it
+//    two free-running waves overlap with MFMAs: 43968 tokens 7.1-7.7 ms
+//    (1.03-1.11 PFLOP/s, boxes differ), 8 x 1374 77 us.
+//  * fine (QB = 1): 32 queries a wave, 157 VGPRs, three 32 KB workgroups a CU.
+//    Twice the LDS reads per MFMA (6-9 % slower on launches of many rounds),
+//    but twice as many workgroups, which fill the CUs of a small launch.  Bound
+//    by the chain QK -> exp2 -> PV of the one or two waves a SIMD then holds.
+//    Against the wide form and 2-wave workgroups of it (what small launches
+//    ran before), same box: 1 x 1374 32 / 29.7 -> 19.8 us, 2 x 1374 33 / 44 ->
+//    28, 4 x 1374 52 / 47 -> 42, 6 x 1374 72 -> 65, 1 x 2748 57 / 78 -> 49,
+//    1 x 4122 127 / 117 -> 98, 1 x 5496 172 / 156 -> 140, 1 x 8244 364 -> 325.
+template <int WAVES, int SUB, int QB>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(QB == 2 ? 2 : 3, QB == 2 ? 2 : 3))) void attention_fwd_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     uint16_t* __restrict__ out, int L, int H, long q_ts, long kv_ts, long v_ts, long o_ts, float scale_log2) {
   constexpr int ATT_WAVES = WAVES;               // waves per workgroup
+  constexpr int ATT_QW = 32 * QB;                // queries per wave
   constexpr int ATT_BQ = ATT_WAVES * ATT_QW;     // queries per workgroup
   constexpr int ATT_SUB = SUB;                   // compute tiles per DMA tile (one barrier per DMA tile)
   constexpr int ATT_BKD = ATT_BK * ATT_SUB;      // keys per DMA tile
@@ -121,10 +130,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
   const bool live = qt * ATT_BQ + wave * ATT_QW < L;   // wave-uniform
 
   // ---- Q^T fragments (B operand of S^T = K Q^T): per query block, 4 k-steps of 16 dims
-  uint4 qf[2][4];
-  int qi[2];
+  uint4 qf[QB][4];
+  int qi[QB];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
     qi[qb] = qt * ATT_BQ + wave * ATT_QW + 32 * qb + l32;     // query index in the sequence
     const int qc = qi[qb] < L ? qi[qb] : L - 1;
     const uint16_t* qp = q + (tok0 + qc) * q_ts + (long)head * 64;
@@ -189,9 +198,9 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
   const int tr_key = 4 * h + ((lane & 15) >> 2);
   const int tr_dim = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
   const int ntiles = (L + ATT_BKD - 1) / ATT_BKD;   // DMA tiles
-  f32x16 o[2][2];   // [query block][dim block]
+  f32x16 o[QB][2];   // [query block][dim block]
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
+  for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
     for (int db = 0; db < 2; ++db)
 #pragma unroll
@@ -204,13 +213,12 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
   // the MFMA's C input), equal to m_use after the first tile, so P = 2^S'
   // needs one exp2 per score and nothing else
   float base[2] = {0.f, 0.f};
-  const f16x2 ones = {(_Float16)1.0f, (_Float16)1.0f};
 
   // one 64-key compute tile: keys key0.., K / V rows at kb_lds / vb
   auto ctile = [&](int key0, const uint8_t* kb_lds, const uint8_t* vb, bool mask) __attribute__((always_inline)) {
     {
       // ---- S^T = K Q^T for the 64 keys of the tile, both query blocks (raw dot products)
-      f32x16 sc[2][2];   // [query block][key block]
+      f32x16 sc[QB][2];   // [query block][key block]
   #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
         const int row = 32 * kb + l32;
@@ -219,7 +227,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
           const int c = 2 * st + h;
           const uint4 kf = *reinterpret_cast<const uint4*>(kb_lds + row * 128 + ((c ^ fk(row)) * 16));
   #pragma unroll
-          for (int qb = 0; qb < 2; ++qb)
+          for (int qb = 0; qb < QB; ++qb)
             sc[qb][kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
                 __builtin_bit_cast(f16x8, kf), __builtin_bit_cast(f16x8, qf[qb][st]),
                 st == 0 ? f32x16{} - base[qb] : sc[qb][kb], 0, 0, 0);
@@ -242,9 +250,9 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
           vfr[db][st] = make_uint4(vv[0].x, vv[0].y, vv[1].x, vv[1].y);
         }
       }
-      uint4 pf[2][4];
+      uint4 pf[QB][4];
   #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) {
+      for (int qb = 0; qb < QB; ++qb) {
         if (mask) {
           const int kh = key0 + 4 * h;
   #pragma unroll
@@ -254,7 +262,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
               if (kh + 32 * kb + 8 * (r >> 2) + (r & 3) >= L) sc[qb][kb][r] = -INFINITY;
         }
         // ---- P = 2^S' = 2^(S - m_use) in fp16 against the current reference,
-        // with this tile's partial row sum t (v_dot2 on the fp16 values).  The
+        // with this tile's partial row sum t (of the fp32 values).  The
         // tile maximum is only needed when some P could exceed 2^RESCALE_SLACK,
         // and every such P makes t exceed it too (P >= 0), so the maximum is
         // computed only for waves where some lane's t does, and on the first
@@ -272,7 +280,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
                 const float p0 = __builtin_amdgcn_exp2f(shift ? s0 + off : s0);
                 const float p1 = __builtin_amdgcn_exp2f(shift ? s1 + off : s1);
                 const f16x2 ph = {(_Float16)p0, (_Float16)p1};
-                t = __builtin_amdgcn_fdot2(ph, ones, t, false);
+                t += p0;
+                t += p1;
                 w[e] = __builtin_bit_cast(uint32_t, ph);
               }
               pf[qb][2 * kb + pp] = make_uint4(w[0], w[1], w[2], w[3]);
@@ -351,7 +360,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
 
   // ---- normalise and store: lane (h, q) holds dims 32db + 8*(r/4) + 4h + r%4
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
     const float l_tot = half_sum(l_run[qb]);
     const float inv = 1.0f / l_tot;
     if (qi[qb] < L) {
@@ -367,6 +376,21 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(2, 2
         }
     }
   }
+}
+
+// Which form a launch of BH (sequence, head) pairs runs, from its estimated
+// time in hundredths of a full wide round (512 workgroups of 256 queries, two
+// a CU).  Wide: whole rounds, then a last one that costs 45 up to one
+// workgroup a CU (64 where it is the only one) and 100 above.  Fine: 82 per
+// 768 workgroups (three a CU) + 13.  Both fitted to the times above and to
+// launches on either side of the line: wide keeps 1 x 6870 (217 against 227
+// us), 1 x 10992 (500 / 527), 8 x 1374 (74 / 77), 16 x 1374 (146 / 146);
+// fine takes 6 x 1374 (72 / 65) and 1 x 8244 (362 / 322).
+static bool attention_fine(long BH, long L) {
+  const long wide = BH * ((L + 255) / 256), fine = BH * ((L + 127) / 128);
+  const long rem = wide % 512;
+  const long wide_cost = wide / 512 * 100 + (rem == 0 ? 0 : rem > 256 ? 100 : wide < 512 ? 64 : 45);
+  return fine * 82 / 768 + 13 < wide_cost;
 }
 
 }  // namespace qv
@@ -387,22 +411,18 @@ extern "C" int qv_attention_fwd(const void* q, const void* k, const void* v, voi
                "q, k, v must be 16-byte and out 8-byte aligned");
   QV_CHECK_ARG((uint64_t)L * k_token_stride * 2 < (1ull << 32) && (uint64_t)L * v_token_stride * 2 < (1ull << 32),
                "sequence too long for 32-bit offsets");
-  // 4-wave workgroups (256 queries) when they fill at least one round of
-  // the 512 workgroup slots (two per CU); else 2-wave workgroups
-  const long qtiles4 = (L + 4 * qv::ATT_QW - 1) / (4 * qv::ATT_QW);
-  const bool wide = B * H * qtiles4 >= 512;
-  const long bq = wide ? 4 * qv::ATT_QW : 2 * qv::ATT_QW;
-  const long nwg = B * H * ((L + bq - 1) / bq);
+  const bool fine = qv::attention_fine(B * H, L);
+  const long nwg = B * H * (fine ? (L + 127) / 128 : (L + 255) / 256);
   QV_CHECK_ARG(nwg <= INT32_MAX, "grid too large");
   const float scale_log2 = scale * 1.4426950408889634f;
 #define QV_ATT_ARGS                                                                                       \
   (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)out, (int)L, (int)H, (long)q_token_stride, \
       (long)k_token_stride, (long)v_token_stride, (long)out_token_stride, scale_log2
-  if (wide)
-    hipLaunchKernelGGL((qv::attention_fwd_kernel<4, 2>), dim3((unsigned)nwg), dim3(256), 0, (hipStream_t)stream,
+  if (fine)
+    hipLaunchKernelGGL((qv::attention_fwd_kernel<4, 1, 1>), dim3((unsigned)nwg), dim3(256), 0, (hipStream_t)stream,
                        QV_ATT_ARGS);
   else
-    hipLaunchKernelGGL((qv::attention_fwd_kernel<2, 1>), dim3((unsigned)nwg), dim3(128), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL((qv::attention_fwd_kernel<4, 2, 2>), dim3((unsigned)nwg), dim3(256), 0, (hipStream_t)stream,
                        QV_ATT_ARGS);
 #undef QV_ATT_ARGS
   return qv::check_launch("attention_fwd");

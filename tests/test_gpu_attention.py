@@ -79,6 +79,25 @@ def test_attention_two_forms_agree_bitwise(gpu):
     assert np.abs(got - ref).max() / np.abs(ref).max() <= TOL
 
 
+@pytest.mark.parametrize("L", [129, 161, 200, 255, 256, 417, 480])
+def test_attention_fine_and_wide_forms_agree_bitwise(gpu, L):
+    """Two sequences alone run 32 queries a wave, the same two at the front of
+    64 run 64 queries a wave: equal bits at lengths that leave part of a wave,
+    whole idle waves or nothing over in either form, and within the tolerance
+    of the oracle."""
+    from qvggt_amd import awq_inference_engine as E
+    H = 16
+    x = _qkv(2 * L, H, 100 + L)
+    xt = torch.from_numpy(x).to(gpu)
+    many = torch.cat([xt, torch.randn(62 * L, 3, H, 64, device=gpu).half()])
+    two = E.attention(xt[:, 0], xt[:, 1], xt[:, 2], L)
+    out = E.attention(many[:, 0], many[:, 1], many[:, 2], L)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:2 * L], two)
+    ref = attention_ref(x[:, 0], x[:, 1], x[:, 2], 2, L)
+    assert np.abs(two.float().cpu().numpy() - ref).max() / np.abs(ref).max() <= TOL
+
+
 def test_attention_separate_buffers_and_determinism(gpu):
     from qvggt_amd import awq_inference_engine as E
     B, L, H = 2, 300, 4
