@@ -322,6 +322,35 @@ int qv_attention_fwd(const void* q, const void* k, const void* v, void* out, int
                      int64_t k_token_stride, int64_t v_token_stride, int64_t out_token_stride,
                      float scale, void* stream);
 
+/* ---------------------------------------------------- camera head
+ * No counterparts in the reference extension: the camera head's graph is in
+ * the external vggt-hf (qvggt/inference/loader.py:204-206 quantises its trunk
+ * linears only). */
+
+/*
+ * Attention over S pose tokens, fp16 in/out, fp32 scores, softmax and sums:
+ * qkv is a contiguous (S, 3, H, 128) buffer, out (S, H, 128);
+ * out = softmax(q k^T * scale) v per head, no mask.  head_dim must be 128.
+ */
+int qv_pose_attention(const void* qkv, void* out, int64_t S, int64_t H, int64_t head_dim,
+                      float scale, void* stream);
+
+/*
+ * x = gate * (adaln * (1 + scale) + shift) + pose in fp32, rounded once to
+ * fp16: mod (S, 3 D) holds shift, scale and gate (D each) a row, the others
+ * are (S, D); D a multiple of 8, everything 16-byte aligned and contiguous.
+ */
+int qv_adaln_modulate(const void* mod, const void* adaln, const void* pose, void* x, int64_t S,
+                      int64_t D, void* stream);
+
+/*
+ * End of a camera-head iteration on (S, cols) values: pred (fp32, in place)
+ * = delta (fp16) if first, else pred + delta; act (fp32) = pred with columns
+ * n_linear and up through ReLU; half (fp16) = pred rounded.
+ */
+int qv_pose_update(const void* delta, float* pred, float* act, void* half, int64_t S, int64_t cols,
+                   int64_t n_linear, int first, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -755,3 +755,49 @@ def qknorm_rope2d(qkv: torch.Tensor, positions: torch.Tensor, cos_table: torch.T
                   cos_table.shape[0], _ptr(qg), _ptr(qb), _ptr(kg), _ptr(kb), C.c_float(eps), T, heads,
                   3 * heads * 64, _stream(dev))
     return qkv
+
+
+# ----------------------------------------------------------- camera head
+def pose_attention(qkv: torch.Tensor, heads: int, scale: float) -> torch.Tensor:
+    """Attention over the S pose tokens of a contiguous (S, 3*heads*128) fp16
+    qkv, in fp32; returns (S, heads*128) fp16."""
+    what = "pose_attention"
+    if qkv.dtype != torch.float16 or qkv.dim() != 2 or qkv.shape[1] != 3 * heads * 128 or not qkv.is_contiguous():
+        _fail(f"{what}: qkv must be contiguous float16 (S, 3*heads*128)")
+    dev = _on_gpu(qkv, what=what)
+    out = torch.empty(qkv.shape[0], heads * 128, dtype=qkv.dtype, device=dev)
+    with _device(dev):
+        _lib.call("qv_pose_attention", _ptr(qkv), _ptr(out), qkv.shape[0], heads, 128, C.c_float(scale), _stream(dev))
+    return out
+
+
+def adaln_modulate(mod: torch.Tensor, adaln: torch.Tensor, pose: torch.Tensor) -> torch.Tensor:
+    """gate * (adaln * (1 + scale) + shift) + pose, mod (S, 3D) = (shift | scale | gate),
+    adaln and pose (S, D), all fp16; evaluated in fp32, rounded once."""
+    what = "adaln_modulate"
+    S, D = adaln.shape
+    for name, t, n in (("mod", mod, 3 * D), ("adaln", adaln, D), ("pose", pose, D)):
+        if t.dtype != torch.float16 or tuple(t.shape) != (S, n):
+            _fail(f"{what}: {name} must be float16 ({S}, {n})")
+    dev = _on_gpu(mod, adaln, pose, what=what)
+    mod, adaln, pose = _contig(mod), _contig(adaln), _contig(pose)
+    x = torch.empty_like(pose)
+    with _device(dev):
+        _lib.call("qv_adaln_modulate", _ptr(mod), _ptr(adaln), _ptr(pose), _ptr(x), S, D, _stream(dev))
+    return x
+
+
+def pose_update(delta: torch.Tensor, pred: torch.Tensor, first: bool, n_linear: int):
+    """pred (S, cols) fp32, in place: delta (fp16) if ``first``, else pred + delta.
+    Returns (pred with columns >= n_linear through ReLU, fp32; pred as fp16)."""
+    what = "pose_update"
+    if delta.dtype != torch.float16 or pred.dtype != torch.float32 or delta.shape != pred.shape or delta.dim() != 2:
+        _fail(f"{what}: delta must be float16 and pred float32, both (S, cols)")
+    _need(pred, torch.float32, what, "pred")
+    dev = _on_gpu(delta, pred, what=what)
+    d = _contig(delta)
+    act, half = torch.empty_like(pred), torch.empty_like(pred, dtype=torch.float16)
+    with _device(dev):
+        _lib.call("qv_pose_update", _ptr(d), _ptr(pred), _ptr(act), _ptr(half), pred.shape[0], pred.shape[1], n_linear,
+                  1 if first else 0, _stream(dev))
+    return act, half

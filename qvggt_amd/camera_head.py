@@ -22,8 +22,8 @@ the trunk blocks, 1e-6 for ``adaln_norm``.
 
 Per frame there is one pose token, so the trunk linears run at M = S: every
 S <= 64 runs on the skinny-M MFMA kernel (through the GEMV entry for
-S <= 16 and the GEMM entry above).  Attention over S tokens with
-head_dim 128 is a few kFLOP and runs in fp32 through torch.
+S <= 16 and the GEMM entry above).  Attention over the S tokens (head_dim
+128, fp32; up to 256 frames), the adaLN modulation and the pose update are one kernel each.
 ``GraphedCameraHead`` records the whole forward as one HIP graph.  The CICT token
 QVGGT's loader can attach (loader.py:224-246) has no public definition and is
 not modelled.
@@ -46,6 +46,10 @@ TRUNK_DEPTH = 4
 POSE_DIM = 9                 # absT (3) + quaternion (4) + FoV (2)
 LN_EPS = 1e-5               # token_norm, trunk_norm, trunk blocks (torch's default)
 ADALN_EPS = 1e-6
+# Frames up to which the pose attention runs in its one fp32 kernel; above, the
+# fp32 batched products of torch are as fast or faster (256 frames: 24 us
+# against 96; 512: 74 / 63; 1024: 262 / 150).
+POSE_ATTENTION_MAX = 256
 
 
 class TrunkBlock(nn.Module):
@@ -68,9 +72,12 @@ class TrunkBlock(nn.Module):
         S = x.shape[0]
         h = E.layer_norm(x, self.norm1.weight, self.norm1.bias, LN_EPS)
         qkv = _linear(self.attn.qkv, h, QV_EPI_BIAS, torch.empty(S, 3 * DIM, dtype=x.dtype, device=x.device))
-        q, k, v = qkv.float().view(S, 3, HEADS, HEAD_DIM).permute(1, 2, 0, 3)   # (H, S, 128) each
-        a = torch.softmax(torch.bmm(q, k.transpose(1, 2).contiguous()) * HEAD_DIM ** -0.5, dim=-1) @ v
-        att = a.permute(1, 0, 2).reshape(S, DIM).half()
+        if S <= POSE_ATTENTION_MAX:
+            att = E.pose_attention(qkv, HEADS, HEAD_DIM ** -0.5)
+        else:
+            q, k, v = qkv.float().view(S, 3, HEADS, HEAD_DIM).permute(1, 2, 0, 3)   # (H, S, 128) each
+            a = torch.softmax(torch.bmm(q, k.transpose(1, 2).contiguous()) * HEAD_DIM ** -0.5, dim=-1) @ v
+            att = a.permute(1, 0, 2).reshape(S, DIM).half()
         _linear_residual(self.attn.proj, att, self.ls1.gamma, x, torch.empty(S, DIM, dtype=x.dtype, device=x.device))
         h = E.layer_norm(x, self.norm2.weight, self.norm2.bias, LN_EPS)
         f = _linear(self.mlp.fc1, h, QV_EPI_BIAS_GELU, torch.empty(S, MLP_DIM, dtype=x.dtype, device=x.device))
@@ -153,24 +160,24 @@ class CameraHead(nn.Module):
         S = tokens.shape[0]
         pose = E.layer_norm(tokens.contiguous(), self.token_norm.weight, self.token_norm.bias, LN_EPS)
         adaln = E.layer_norm(pose, self._ones, self._zeros, ADALN_EPS)
-        pred, outs = None, []
-        for _ in range(num_iterations):
-            src = self.empty_pose_tokens.view(1, POSE_DIM).expand(S, POSE_DIM) if pred is None else pred.half()
-            mod = self.poseLN_modulation(self.embed_pose(src))
-            shift, scale, gate = mod.chunk(3, dim=-1)
-            x = (gate * (adaln * (1 + scale) + shift) + pose).contiguous()
+        # the first iteration embeds empty_pose_tokens, the later ones the prediction
+        src = self.empty_pose_tokens.view(1, POSE_DIM).expand(S, POSE_DIM)
+        pred = torch.empty(S, POSE_DIM, dtype=torch.float32, device=tokens.device)
+        outs = []
+        for i in range(num_iterations):
+            x = E.adaln_modulate(self.poseLN_modulation(self.embed_pose(src)), adaln, pose)
             for blk in self.trunk:
                 blk(x)
             h = E.layer_norm(x, self.trunk_norm.weight, self.trunk_norm.bias, LN_EPS)
-            delta = self.pose_branch.fc2(F.gelu(self.pose_branch.fc1(h))).float()
-            pred = delta if pred is None else pred + delta
-            outs.append(self.activate(pred))
+            delta = self.pose_branch.fc2(F.gelu(self.pose_branch.fc1(h)))
+            act, src = E.pose_update(delta, pred, i == 0, 7)
+            outs.append(act)
         return outs
 
 
 class GraphedCameraHead:
     """``CameraHead.forward`` for a fixed frame count S, recorded once as a HIP
-    graph and replayed: the head is ~400 small launches per call (4 iterations
+    graph and replayed: the head is ~150 small launches per call (4 iterations
     x 4 trunk blocks of LayerNorm, four W4 linears at M = S, attention and
     residual updates), so replay removes the host launch cost that otherwise
     dominates at small S.  ``__call__(tokens)`` copies ``tokens`` (S, 2048)

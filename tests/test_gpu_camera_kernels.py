@@ -1,0 +1,71 @@
+"""The camera head's small kernels against torch in float64.
+
+Bounds: the kernels compute in fp32 and round once to fp16, so an output is
+within half an fp16 step (2^-11 relative, 2^-25 absolute below the normal
+range) of the exact value plus the fp32 error of the sums, which 1e-5 of the
+largest term covers (under 300 terms at 6e-8 each).
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(got, ref, scale):
+    got, ref = got.double(), ref.double()
+    assert torch.isfinite(got).all()
+    assert ((got - ref).abs() <= ref.abs() * 2.0 ** -11 + 2.0 ** -25 + 1e-5 * scale).all()
+
+
+@pytest.mark.parametrize("S", [1, 3, 4, 5, 16, 17, 63, 64, 65, 127, 129, 200])
+@pytest.mark.parametrize("H,sigma", [(16, 1.0), (3, 6.0)])
+def test_pose_attention(gpu, S, H, sigma):
+    """Around the query blocks (4), the 64-key tiles and their
+    remainders; sigma = 6 spreads the scores over hundreds, so the running
+    maximum moves between tiles."""
+    from qvggt_amd import awq_inference_engine as E
+    g = torch.Generator(device=gpu).manual_seed(S)
+    qkv = (torch.randn(S, 3, H, 128, generator=g, device=gpu) * sigma).half()
+    out = E.pose_attention(qkv.view(S, -1), H, 128 ** -0.5)
+    q, k, v = (qkv[:, i].double().transpose(0, 1).contiguous() for i in range(3))
+    s = q @ k.transpose(1, 2).contiguous() * 128 ** -0.5
+    ref = (torch.softmax(s, -1) @ v).transpose(0, 1).reshape(S, H * 128)
+    # an fp32 score is off by up to ~1e-6 of the largest, and p by that factor
+    _close(out, ref, v.abs().max().item() * max(1.0, s.abs().max().item() / 5))
+
+
+@pytest.mark.parametrize("S,D", [(1, 8), (3, 2048), (80, 2048), (5, 264)])
+def test_adaln_modulate(gpu, S, D):
+    from qvggt_amd import awq_inference_engine as E
+    g = torch.Generator(device=gpu).manual_seed(S + D)
+    mod, a, p = (torch.randn(S, n, generator=g, device=gpu).half() for n in (3 * D, D, D))
+    x = E.adaln_modulate(mod, a, p)
+    sh, sc, ga = mod.double().chunk(3, -1)
+    _close(x, ga * (a.double() * (1 + sc) + sh) + p.double(), 1.0)
+    wide = torch.randn(S, 3 * D + 8, generator=g, device=gpu).half()
+    wide[:, :3 * D] = mod
+    assert torch.equal(E.adaln_modulate(wide[:, :3 * D], a, p), x)      # a strided input
+
+
+@pytest.mark.parametrize("S", [1, 28, 29, 300])
+def test_pose_update(gpu, S):
+    """Exact: the fp32 add, ReLU (NaN stays) and the rounding to fp16."""
+    from qvggt_amd import awq_inference_engine as E
+    g = torch.Generator(device=gpu).manual_seed(S)
+    pred = torch.full((S, 9), float("nan"), device=gpu)
+    want = None
+    for i in range(3):
+        d = torch.randn(S, 9, generator=g, device=gpu).half()
+        if i == 2:
+            d[0, 8], d[0, 0] = float("nan"), float("inf")
+        want = d.float() if want is None else want + d.float()
+        act, half = E.pose_update(d, pred, i == 0, 7)
+        ref = torch.cat([want[:, :7], torch.relu(want[:, 7:])], -1)
+        assert torch.equal(act.nan_to_num(123.0), ref.nan_to_num(123.0))
+        assert torch.equal(half.nan_to_num(123.0), want.half().nan_to_num(123.0))
+        assert torch.equal(pred.nan_to_num(123.0), want.nan_to_num(123.0))
+
+
+def test_empty(gpu):
+    from qvggt_amd import awq_inference_engine as E
+    assert E.pose_attention(torch.empty(0, 6144, device=gpu, dtype=torch.float16), 16, 0.1).shape == (0, 2048)
