@@ -43,7 +43,7 @@ import torch.nn.functional as F
 
 from . import awq_inference_engine as E
 from ._lib import QV_EPI_BIAS, QV_EPI_BIAS_GELU
-from .awq.qmodule import WQLinear
+from .awq.qmodule import WQLinear, w4_buffers
 
 GRID = 37
 PATCH = 14
@@ -239,9 +239,11 @@ def _linear_residual(layer, x: torch.Tensor, gamma: torch.Tensor, resid: torch.T
     """resid += gamma * layer(x): a block's proj / fc2 with its LayerScale
     residual update, fused into the W4A16 epilogue when the layer is a
     ``WQLinear`` with a bias; otherwise the linear, then torch's addcmul."""
-    if isinstance(layer, WQLinear) and layer.bias is not None:
-        E.w4a16_linear_residual(x, layer.qweight, layer.scales, layer.scaled_zeros, layer.bias, gamma, resid)
-        return resid
+    if isinstance(layer, WQLinear):
+        qweight, scales, scaled_zeros, bias = w4_buffers(layer)
+        if bias is not None:
+            E.w4a16_linear_residual(x, qweight, scales, scaled_zeros, bias, gamma, resid)
+            return resid
     o = _linear(layer, x, QV_EPI_BIAS if layer.bias is not None else 0, out)
     return resid.addcmul_(o, gamma)
 
@@ -251,8 +253,8 @@ def _linear(layer, x: torch.Tensor, epilogue: int, out: torch.Tensor) -> torch.T
     bias (+ GELU) fused, or an unquantised fp16 ``nn.Linear`` (blocks a
     checkpoint leaves in floating point, loader.py:320-362) through torch."""
     if isinstance(layer, WQLinear):
-        return E.w4a16_linear(x, layer.qweight, layer.scales, layer.scaled_zeros, bias=layer.bias,
-                              epilogue=epilogue, out=out)
+        qweight, scales, scaled_zeros, bias = w4_buffers(layer)
+        return E.w4a16_linear(x, qweight, scales, scaled_zeros, bias=bias, epilogue=epilogue, out=out)
     if layer.bias is not None:
         y = torch.addmm(layer.bias, x, layer.weight.t(), out=out)
     else:
@@ -260,6 +262,15 @@ def _linear(layer, x: torch.Tensor, epilogue: int, out: torch.Tensor) -> torch.T
     if epilogue == QV_EPI_BIAS_GELU:
         y.copy_(F.gelu(y))
     return y
+
+
+def _affine(ln: nn.LayerNorm):
+    """A norm's (weight, bias), read from its parameter table (see ``w4_buffers``)."""
+    p = ln._parameters
+    try:
+        return p["weight"], p["bias"]
+    except KeyError:    # parametrised
+        return ln.weight, ln.bias
 
 
 def _with_depth(cfg: AggregatorConfig, depth: int | None) -> AggregatorConfig:
@@ -306,41 +317,42 @@ class AABlock(nn.Module):
     def forward(self, x: torch.Tensor, seq_len: int, pos: torch.Tensor, tables, ws: dict) -> torch.Tensor:
         """x: (M, 1024) fp16, updated in place.  ws: scratch buffers keyed by name."""
         M = x.shape[0]
-        a = self.attn
-        eps = self.eps
-        if not self.w8a8 and isinstance(a.qkv, WQLinear) and a.qkv.bias is not None:
+        a, m = self.attn, self.mlp
+        wqkv, proj, q_norm, k_norm = a.qkv, a.proj, _affine(a.q_norm), _affine(a.k_norm)
+        n1, n2, gamma1, gamma2 = _affine(self.norm1), _affine(self.norm2), self.ls1.gamma, self.ls2.gamma
+        eps, w8a8 = self.eps, self.w8a8
+        qweight, scales, scaled_zeros, bias = (w4_buffers(wqkv) if not w8a8 and isinstance(wqkv, WQLinear)
+                                               else (None,) * 4)
+        if bias is not None:
             # the qkv projection with its q/k LayerNorm and 2-D RoPE in the GEMM epilogue
-            h = E.layer_norm(x, self.norm1.weight, self.norm1.bias, eps, out=ws["h"])
-            qkv = E.w4a16_linear_qkrope(h, a.qkv.qweight, a.qkv.scales, a.qkv.scaled_zeros, a.qkv.bias, pos,
-                                        tables[0], tables[1], HEADS, a.q_norm.weight, a.q_norm.bias,
-                                        a.k_norm.weight, a.k_norm.bias, eps, out=ws["qkv"])
+            h = E.layer_norm(x, *n1, eps, out=ws["h"])
+            qkv = E.w4a16_linear_qkrope(h, qweight, scales, scaled_zeros, bias, pos, tables[0], tables[1], HEADS,
+                                        *q_norm, *k_norm, eps, out=ws["qkv"])
         else:
-            if not self.w8a8:
-                h = E.layer_norm(x, self.norm1.weight, self.norm1.bias, eps, out=ws["h"])
-                qkv = _linear(a.qkv, h, QV_EPI_BIAS, ws["qkv"])
+            if not w8a8:
+                h = E.layer_norm(x, *n1, eps, out=ws["h"])
+                qkv = _linear(wqkv, h, QV_EPI_BIAS, ws["qkv"])
             else:
-                E.rms_norm_general(ws["q8"], x, self.norm1.weight, self.norm1.bias, ws["s8"], eps, True)
-                qkv = a.qkv(ws["q8"], ws["s8"], out=ws["qkv"])
-            E.qknorm_rope2d(qkv, pos, tables[0], tables[1], HEADS, a.q_norm.weight, a.q_norm.bias,
-                            a.k_norm.weight, a.k_norm.bias, eps)
+                E.rms_norm_general(ws["q8"], x, *n1, ws["s8"], eps, True)
+                qkv = wqkv(ws["q8"], ws["s8"], out=ws["qkv"])
+            E.qknorm_rope2d(qkv, pos, tables[0], tables[1], HEADS, *q_norm, *k_norm, eps)
         v3 = qkv.view(M, 3, HEADS, HEAD_DIM)
-        att = E.attention(v3[:, 0], v3[:, 1], v3[:, 2], seq_len, out=ws["att"].view(M, HEADS, HEAD_DIM))
+        att = E.attention(*v3.unbind(1), seq_len, out=ws["att"].view(M, HEADS, HEAD_DIM))
         att = att.view(M, DIM)
-        if not self.w8a8:
-            _linear_residual(a.proj, att, self.ls1.gamma, x, ws["o"])
+        if not w8a8:
+            _linear_residual(proj, att, gamma1, x, ws["o"])
         else:
             E.invoke_quant(ws["q8"], att, ws["s8"])
-            a.proj.forward_residual(ws["q8"], ws["s8"], self.ls1.gamma, x)
-        m = self.mlp
-        if not self.w8a8:
-            h = E.layer_norm(x, self.norm2.weight, self.norm2.bias, eps, out=ws["h"])
+            proj.forward_residual(ws["q8"], ws["s8"], gamma1, x)
+        if not w8a8:
+            h = E.layer_norm(x, *n2, eps, out=ws["h"])
             f = _linear(m.fc1, h, QV_EPI_BIAS_GELU, ws["f"])
-            _linear_residual(m.fc2, f, self.ls2.gamma, x, ws["o"])
+            _linear_residual(m.fc2, f, gamma2, x, ws["o"])
         else:
-            E.rms_norm_general(ws["q8"], x, self.norm2.weight, self.norm2.bias, ws["s8"], eps, True)
+            E.rms_norm_general(ws["q8"], x, *n2, ws["s8"], eps, True)
             f = m.fc1(ws["q8"], ws["s8"], out=ws["f"])
             E.gelu_and_quant(ws["q8f"], f, ws["s8"], None)   # the fp16 GELU copy is not needed
-            m.fc2.forward_residual(ws["q8f"], ws["s8"], self.ls2.gamma, x)
+            m.fc2.forward_residual(ws["q8f"], ws["s8"], gamma2, x)
         return x
 
 
@@ -533,6 +545,7 @@ class Aggregator(nn.Module):
                 "h": torch.empty(M, DIM, **f16), "qkv": torch.empty(M, 3 * DIM, **f16),
                 "att": torch.empty(M, DIM, **f16), "o": torch.empty(M, DIM, **f16),
                 "f": torch.empty(M, MLP_DIM, **f16),
+                "pos": vggt_positions(M // TOKENS, dev),
             }
             if self.w8a8:
                 self._ws.update({
@@ -550,7 +563,7 @@ class Aggregator(nn.Module):
         ws = self._workspace(M, dev)
         if self._tables is None or self._tables[0].device != dev:
             self._tables = E.rope2d_tables(GRID + 1, self.config.rope_base, device=dev)
-        pos = vggt_positions(S, dev)
+        pos = ws["pos"]
         x_img = (images - self.img_mean) / self.img_std
         patches = self.patch_embed(x_img, ws)                                   # (S, 1369, D)
         x = torch.empty(S, TOKENS, DIM, dtype=torch.float16, device=dev)

@@ -60,6 +60,16 @@ def pack_intweight(unpacked_qweight: torch.Tensor, interleave: int, kstride: int
     return packed.to(torch.int16).contiguous()
 
 
+def w4_buffers(layer: "WQLinear"):
+    """(qweight, scales, scaled_zeros, bias) of a ``WQLinear``, read from its
+    buffer table (``nn.Module.__getattr__`` costs about a microsecond each)."""
+    b = layer._buffers
+    try:
+        return b["qweight"], b["scales"], b["scaled_zeros"], b["bias"] if "bias" in b else layer.bias
+    except KeyError:    # a buffer replaced by something of another kind
+        return layer.qweight, layer.scales, layer.scaled_zeros, layer.bias
+
+
 class ScaledActivation(nn.Module):
     """act(x) / scales (qmodule.py:101-113)."""
 
@@ -150,9 +160,9 @@ class WQLinear(nn.Module):
         if self.group_size != 128:
             raise RuntimeError(f"WQLinear.forward: group size {self.group_size} unsupported "
                                "(the reference kernels hard-code 128)")
-        epi = QV_EPI_BIAS if self.bias is not None else QV_EPI_NONE
-        return engine.w4a16_linear(x, self.qweight, self.scales, self.scaled_zeros,
-                                   bias=self.bias, epilogue=epi)
+        qweight, scales, scaled_zeros, bias = w4_buffers(self)
+        return engine.w4a16_linear(x, qweight, scales, scaled_zeros, bias=bias,
+                                   epilogue=QV_EPI_BIAS if bias is not None else QV_EPI_NONE)
 
     def extra_repr(self) -> str:
         return "in_features={}, out_features={}, bias={}, w_bit={}, group_size={}".format(

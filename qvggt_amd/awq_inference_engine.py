@@ -50,38 +50,39 @@ def _dtype_code(t: torch.Tensor, what: str) -> int:
     _fail(f"{what}: failed to dispatch data type {t.dtype} (expected float16 or bfloat16)")
 
 
-def _on_gpu(*tensors: torch.Tensor, what: str):
-    dev = None
+def _on_gpu(*tensors: torch.Tensor, what: str) -> int:
+    """The index of the one GPU that all the tensors (None aside) are on."""
+    dev = -1
     for t in tensors:
         if t is None:
             continue
         if not isinstance(t, torch.Tensor):
             _fail(f"{what}: expected a tensor, got {type(t).__name__}")
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             _fail(f"{what}: tensor on {t.device}; this op runs on the GPU only (no CPU path)")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            _fail(f"{what}: tensors on different devices ({dev} vs {t.device})")
+        d = t.get_device()
+        if d != dev:
+            if dev >= 0:
+                _fail(f"{what}: tensors on different devices (cuda:{dev} vs {t.device})")
+            dev = d
     return dev
 
 
+# The call path of an op is Python, so its cost (17 us for a linear when each
+# pointer and the stream were wrapped in objects, 8-9 us now) bounds small launches: the
+# pointers, the stream and the device go to ctypes as plain integers.
 def _ptr(t: torch.Tensor | None):
-    return C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(0)
+    return t.data_ptr() if t is not None else None
 
 
-def _stream(dev: torch.device):
-    return C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-
-
+_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)   # device index -> the current stream's handle
+_current_device = getattr(torch._C, "_cuda_getDevice", None)     # (a torch without GPU support has neither)
 _NULLCTX = contextlib.nullcontext()
 
 
-def _device(dev: torch.device):
+def _device(dev: int):
     """Device guard; free when ``dev`` is already the current device."""
-    if dev.index is None or dev.index == torch.cuda.current_device():
-        return _NULLCTX
-    return torch.cuda.device(dev)
+    return _NULLCTX if dev == _current_device() else torch.cuda.device(dev)
 
 
 def _contig(t: torch.Tensor) -> torch.Tensor:
@@ -125,12 +126,14 @@ def _check_w4_tables(kernel, scales, zeros, N, K, dt, what):
     if kernel.numel() * kernel.element_size() != N * K // 2:
         _fail(f"{what}: packed weight holds {kernel.numel() * kernel.element_size()} bytes, "
               f"expected N*K/2 = {N * K // 2}")
-    for name, t in (("scales", scales), ("zeros", zeros)):
-        if t.dtype != dt:
-            _fail(f"{what}: {name} dtype {t.dtype} != input dtype {dt}")
-        if t.dim() != 2 or t.shape[1] != N or t.shape[0] < K // GROUP_SIZE:
-            _fail(f"{what}: {name} must be (rows >= K/128 = {K // GROUP_SIZE}, N = {N}), "
-                  f"got {tuple(t.shape)}")
+    rows = K // GROUP_SIZE
+    for t in (scales, zeros):
+        sh = t.shape
+        if t.dtype != dt or len(sh) != 2 or sh[1] != N or sh[0] < rows:
+            name = "scales" if t is scales else "zeros"
+            if t.dtype != dt:
+                _fail(f"{what}: {name} dtype {t.dtype} != input dtype {dt}")
+            _fail(f"{what}: {name} must be (rows >= K/128 = {rows}, N = {N}), got {tuple(sh)}")
 
 
 # ----------------------------------------------------------- W4A16 GEMM/GEMV
@@ -157,7 +160,7 @@ def w4a16_linear(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
     dev = _on_gpu(x, qweight, scales, scaled_zeros, bias, out, what=what)
     x = _contig(x)
     if out is None:
-        out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=dev)
+        out = x.new_empty((*x.shape[:-1], N))
     # contiguous copies bound to names: they must outlive the native call
     qw, sc, sz, bb = _contig(qweight), _contig(scales), _contig(scaled_zeros), _contig_opt(bias)
     with _device(dev):
@@ -201,7 +204,7 @@ def w4a16_linear_qkrope(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Te
                   k_gamma, k_beta, out, what=what)
     x = _contig(x)
     if out is None:
-        out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=dev)
+        out = x.new_empty((*x.shape[:-1], N))
     # contiguous copies bound to names: they must outlive the native call
     qw, sc, sz, bb = _contig(qweight), _contig(scales), _contig(scaled_zeros), _contig(bias)
     pos = _contig(positions)
@@ -209,7 +212,7 @@ def w4a16_linear_qkrope(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Te
     with _device(dev):
         _lib.call("qv_w4a16_gemm_qkrope", _ptr(x), _ptr(qw), _ptr(sc), _ptr(sz), _ptr(bb), _ptr(out), M, N, K,
                   _ptr(pos), _ptr(cos_table), _ptr(sin_table), cos_table.shape[0], _ptr(qg), _ptr(qb), _ptr(kg),
-                  _ptr(kb), C.c_float(eps), heads, _stream(dev))
+                  _ptr(kb), eps, heads, _stream(dev))
     return out
 
 
@@ -267,12 +270,12 @@ def gemm_forward_cuda_new(in_feats: torch.Tensor, kernel: torch.Tensor, scales: 
     _check_w4_tables(kernel, scales, zeros, N, K, in_feats.dtype, what)
     dev = _on_gpu(in_feats, kernel, scales, zeros, what=what)
     x = _contig(in_feats)
-    out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=dev)
+    out = x.new_empty((*x.shape[:-1], N))
     if M == 0:
         return out
     qw, sc, sz = _contig(kernel), _contig(scales), _contig(zeros)
     with _device(dev):
-        _lib.call("qv_w4a16_gemm", _ptr(x), _ptr(qw), _ptr(sc), _ptr(sz), C.c_void_p(0), _ptr(out),
+        _lib.call("qv_w4a16_gemm", _ptr(x), _ptr(qw), _ptr(sc), _ptr(sz), None, _ptr(out),
                   M, N, K, dt, QV_EPI_NONE, _stream(dev))
     return out
 
@@ -299,10 +302,10 @@ def gemv_forward_cuda_new(in_feats: torch.Tensor, kernel: torch.Tensor,
     _check_w4_tables(kernel, scaling_factors, zeros, n, k, in_feats.dtype, what)
     dev = _on_gpu(in_feats, kernel, scaling_factors, zeros, what=what)
     x = _contig(in_feats)
-    out = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=dev)
+    out = x.new_empty((*x.shape[:-1], n))
     qw, sc, sz = _contig(kernel), _contig(scaling_factors), _contig(zeros)
     with _device(dev):
-        _lib.call("qv_w4a16_gemv", _ptr(x), _ptr(qw), _ptr(sc), _ptr(sz), C.c_void_p(0), _ptr(out),
+        _lib.call("qv_w4a16_gemv", _ptr(x), _ptr(qw), _ptr(sc), _ptr(sz), None, _ptr(out),
                   m, n, k, group_size, dt, QV_EPI_NONE, _stream(dev))
     return out
 
@@ -560,7 +563,7 @@ def rms_norm_general(out: torch.Tensor, input: torch.Tensor, weight: torch.Tenso
     b = _contig(bias) if use_per_token_quant else None
     with _device(dev):
         _lib.call("qv_layernorm_quant", _ptr(x), dt, _ptr(w), _ptr(b), _ptr(out), _ptr(scaling),
-                  C.c_float(epsilon), 1 if use_per_token_quant else 0, M, D, _stream(dev))
+                  epsilon, 1 if use_per_token_quant else 0, M, D, _stream(dev))
 
 
 def gelu_and_quant(out: torch.Tensor, input: torch.Tensor, scale_out: torch.Tensor, tmp: torch.Tensor | None) -> None:
@@ -601,7 +604,7 @@ def layernorm_forward_cuda(_input: torch.Tensor, _gamma: torch.Tensor, _out: tor
     dev = _on_gpu(_input, _gamma, _out, what=what)
     x, g = _contig(_input), _contig(_gamma)
     with _device(dev):
-        _lib.call("qv_rmsnorm", _ptr(x), _ptr(g), _ptr(_out), C.c_float(eps), M, D, dt, _stream(dev))
+        _lib.call("qv_rmsnorm", _ptr(x), _ptr(g), _ptr(_out), eps, M, D, dt, _stream(dev))
 
 
 def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: float = 1e-6,
@@ -621,7 +624,7 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: f
     elif out.dtype != x.dtype or out.numel() != x.numel() or not out.is_contiguous():
         _fail(f"{what}: out must be a contiguous {x.dtype} tensor of {x.numel()} elements")
     with _device(dev):
-        _lib.call("qv_layernorm", _ptr(x), _ptr(w), _ptr(b), _ptr(out), C.c_float(eps), M, D, dt,
+        _lib.call("qv_layernorm", _ptr(x), _ptr(w), _ptr(b), _ptr(out), eps, M, D, dt,
                   _stream(dev))
     return out
 
@@ -728,7 +731,7 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, seq_len: int, s
         _fail(f"{what}: out must be float16 (T, H, 64) with head stride 64")
     with _device(dev):
         _lib.call("qv_attention_fwd", _ptr(q), _ptr(k), _ptr(v), _ptr(out), T // seq_len, seq_len, H, 64,
-                  q.stride(0), k.stride(0), v.stride(0), out.stride(0), C.c_float(scale), _stream(dev))
+                  q.stride(0), k.stride(0), v.stride(0), out.stride(0), scale, _stream(dev))
     return out
 
 
@@ -752,7 +755,7 @@ def qknorm_rope2d(qkv: torch.Tensor, positions: torch.Tensor, cos_table: torch.T
     qg, qb, kg, kb = _contig(q_gamma), _contig(q_beta), _contig(k_gamma), _contig(k_beta)
     with _device(dev):
         _lib.call("qv_qknorm_rope2d", _ptr(qkv), _ptr(pos), _ptr(cos_table), _ptr(sin_table),
-                  cos_table.shape[0], _ptr(qg), _ptr(qb), _ptr(kg), _ptr(kb), C.c_float(eps), T, heads,
+                  cos_table.shape[0], _ptr(qg), _ptr(qb), _ptr(kg), _ptr(kb), eps, T, heads,
                   3 * heads * 64, _stream(dev))
     return qkv
 
@@ -767,7 +770,7 @@ def pose_attention(qkv: torch.Tensor, heads: int, scale: float) -> torch.Tensor:
     dev = _on_gpu(qkv, what=what)
     out = torch.empty(qkv.shape[0], heads * 128, dtype=qkv.dtype, device=dev)
     with _device(dev):
-        _lib.call("qv_pose_attention", _ptr(qkv), _ptr(out), qkv.shape[0], heads, 128, C.c_float(scale), _stream(dev))
+        _lib.call("qv_pose_attention", _ptr(qkv), _ptr(out), qkv.shape[0], heads, 128, scale, _stream(dev))
     return out
 
 

@@ -36,7 +36,7 @@ import torch.nn.functional as F
 
 from . import awq_inference_engine as E
 from ._lib import QV_EPI_BIAS, QV_EPI_BIAS_GELU
-from .aggregator import LayerScale, Mlp, _linear, _linear_residual, quantize_w4
+from .aggregator import LayerScale, Mlp, _affine, _linear, _linear_residual, quantize_w4
 
 DIM = 2048
 HEADS = 16
@@ -70,18 +70,20 @@ class TrunkBlock(nn.Module):
     @torch.no_grad()
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         S = x.shape[0]
-        h = E.layer_norm(x, self.norm1.weight, self.norm1.bias, LN_EPS)
-        qkv = _linear(self.attn.qkv, h, QV_EPI_BIAS, torch.empty(S, 3 * DIM, dtype=x.dtype, device=x.device))
+        attn, mlp = self.attn, self.mlp
+        h = E.layer_norm(x, *_affine(self.norm1), LN_EPS)
+        qkv = _linear(attn.qkv, h, QV_EPI_BIAS, x.new_empty((S, 3 * DIM)))
         if S <= POSE_ATTENTION_MAX:
             att = E.pose_attention(qkv, HEADS, HEAD_DIM ** -0.5)
         else:
             q, k, v = qkv.float().view(S, 3, HEADS, HEAD_DIM).permute(1, 2, 0, 3)   # (H, S, 128) each
             a = torch.softmax(torch.bmm(q, k.transpose(1, 2).contiguous()) * HEAD_DIM ** -0.5, dim=-1) @ v
             att = a.permute(1, 0, 2).reshape(S, DIM).half()
-        _linear_residual(self.attn.proj, att, self.ls1.gamma, x, torch.empty(S, DIM, dtype=x.dtype, device=x.device))
-        h = E.layer_norm(x, self.norm2.weight, self.norm2.bias, LN_EPS)
-        f = _linear(self.mlp.fc1, h, QV_EPI_BIAS_GELU, torch.empty(S, MLP_DIM, dtype=x.dtype, device=x.device))
-        _linear_residual(self.mlp.fc2, f, self.ls2.gamma, x, torch.empty(S, DIM, dtype=x.dtype, device=x.device))
+        o = x.new_empty((S, DIM))   # for a linear that is not fused with its residual update
+        _linear_residual(attn.proj, att, self.ls1.gamma, x, o)
+        h = E.layer_norm(x, *_affine(self.norm2), LN_EPS)
+        f = _linear(mlp.fc1, h, QV_EPI_BIAS_GELU, x.new_empty((S, MLP_DIM)))
+        _linear_residual(mlp.fc2, f, self.ls2.gamma, x, o)
         return x
 
 
