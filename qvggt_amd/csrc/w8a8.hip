@@ -15,6 +15,10 @@
 // K-slots: k-step s (0..1) of a stage, lane half h: k = 32*s + 16*h + 0..15
 // (16 contiguous bytes = chunk 2s + h) on both operands.  Output: lane (h, l),
 // register r holds out[m = l][n = 8*(r/4) + 4*h + r%4] of the wave's tile.
+// K split (KSP = 2): two 4-wave groups of one 8-wave workgroup run the main
+// loop over half the stages each, in stage buffers of their own, so that in a
+// launch of at most one tile a CU each SIMD holds a wave of either group;
+// group 1 then hands its int32 sums to group 0 through LDS (exact).
 // Packed weights (PACKED, qv_w8a8_gemm_packed): the weights are re-laid out
 // once (qv_w8a8_pack_weight) so that the 16-byte B fragment of lane L for
 // column block cb (32 channels), stage ks and k-step s sits at byte
@@ -41,8 +45,9 @@ __device__ __forceinline__ int f8(int r) { return (r + (r >> 2)) & 3; }
 
 // OUT: 0 = fp16 (scaled), 1 = fp16 (scaled + bias), 2 = raw int32,
 // 3 = fp16 (scaled + bias) LayerScale-added to `out` in place
-template <int MT, int OUT, bool PACKED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+// KSP: 1, or 2 = K split between two 4-wave groups of one 8-wave workgroup
+template <int MT, int OUT, bool PACKED, int KSP>
+__global__ __launch_bounds__(256 * KSP) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b,
                       const uint16_t* __restrict__ ws, const uint16_t* __restrict__ as,
                       const uint16_t* __restrict__ bias, const uint16_t* __restrict__ gamma,
@@ -52,13 +57,19 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
   constexpr int A_BYTES = BM * 64, B_BYTES = PACKED ? 0 : BN * 64;
   constexpr int STAGE = A_BYTES + B_BYTES;
   constexpr int NSTAGE = 3;
-  constexpr int A_INSTR = BM / 64;   // 1 KB direct loads per wave per stage (A)
+  constexpr int A_BLK = BM / 16;             // 1 KB (16-row) blocks of A a stage
+  constexpr int A_INSTR = (A_BLK + 3) / 4;   // direct loads per wave per stage (A; past A_BLK the last block again)
   constexpr int B_INSTR = 4;         // 16 KB / 1 KB / 4 waves (LDS path)
   constexpr int EP = 128;            // bytes per staged epilogue row (64 fp16, chunk-swizzled: stg_off)
-  constexpr int LDS_BYTES = NSTAGE * STAGE > 4 * BM * EP ? NSTAGE * STAGE : 4 * BM * EP;
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_BYTES];
+  constexpr int GROUP = (PACKED && KSP == 2 ? 4 : NSTAGE) * STAGE;   // stage buffers of a wave group
+  constexpr int PART = KSP == 2 ? BM * BN * 4 : 0;                  // group 1's int32 partial sums
+  constexpr int LDS_MIN = GROUP * KSP > PART ? GROUP * KSP : PART;
+  constexpr int LDS_BYTES = LDS_MIN > 4 * BM * EP ? LDS_MIN : 4 * BM * EP;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds_all[LDS_BYTES];
 
-  const int tid = threadIdx.x;
+  const int grp = KSP == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
+  uint8_t* const lds = lds_all + grp * GROUP;
+  const int tid = threadIdx.x & 255;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, l32 = lane & 31;
@@ -73,7 +84,8 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
   const int gw = tiles_n - g * gn < gn ? tiles_n - g * gn : gn;
   const int m0 = (r / gw) * BM;
   const int n0 = (g * gn + r % gw) * BN;
-  const int KS = K >> 6;
+  const int KS = (K >> 6) / KSP;   // stages of a group: [k_off, k_off + KS)
+  const int k_off = grp * KS;
 
   // The epilogue's per-channel scales / bias and per-token scales, loaded
   // before the main loop so their latency hides under it (read after the
@@ -83,7 +95,7 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
   // (measured, mean of four same-process A/B runs: fc1 at 10,992 tokens
   // -2.2 %, qkv at 10,992 tokens -3.1 %; qkv at 1,374 tokens +2 % when the
   // 64-row tiles prefetched too).
-  constexpr bool PREF = OUT != 2 && MT >= 4;
+  constexpr bool PREF = OUT != 2 && MT >= 4 && KSP == 1;
   uint2 wsv[NT][4], bsv[NT][4];
   uint16_t asv[MT];
   if constexpr (PREF) {
@@ -121,14 +133,15 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
     const uint32_t base = lds0 + st * STAGE;
 #pragma unroll
     for (int q = 0; q < A_INSTR; ++q) {
-      const int r0 = 16 * (A_INSTR * wave + q);
-      lds_dma16(rsA, voff[(r0 >> 4) & 1], r0 * K + ks * 64, base + r0 * 64);
+      const int b = A_INSTR * wave + q;
+      const int r0 = 16 * (A_BLK % 4 == 0 || b < A_BLK ? b : A_BLK - 1);
+      lds_dma16(rsA, voff[(r0 >> 4) & 1], r0 * K + (k_off + ks) * 64, base + r0 * 64);
     }
     if constexpr (!PACKED) {
 #pragma unroll
       for (int q = 0; q < B_INSTR; ++q) {
         const int r0 = 16 * (B_INSTR * wave + q);
-        lds_dma16(rsB, voff[(r0 >> 4) & 1], r0 * K + ks * 64, base + A_BYTES + r0 * 64);
+        lds_dma16(rsB, voff[(r0 >> 4) & 1], r0 * K + (k_off + ks) * 64, base + A_BYTES + r0 * 64);
       }
     }
   };
@@ -159,7 +172,7 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
       for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2)
-          bw[j][s2] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsB, b_voff[j], ks * 2048 + 1024 * s2, 0));
+          bw[j][s2] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsB, b_voff[j], (k_off + ks) * 2048 + 1024 * s2, 0));
     };
     auto mfmas = [&](const uint4 (&bw)[NT][2], int s, const uint4 (&av)[MT]) {
 #pragma unroll
@@ -205,7 +218,7 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
     constexpr int W_OPS = 2 * NT;              // weight loads per stage
     constexpr int WAIT_TOP = 0x0F70 | (A_INSTR + W_OPS);
     static_assert(A_INSTR + W_OPS < 16, "vmcnt immediate");
-    static_assert(NB * STAGE <= LDS_BYTES, "the activation buffers fit the LDS allocation");
+    static_assert(NB * STAGE <= (KSP == 1 ? LDS_BYTES : GROUP), "the activation buffers fit the LDS allocation");
     uint4 bw3[3][NT][2];
     const int last = KS - 1;
     issue(0, 0);
@@ -299,6 +312,41 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
     }
   }
 
+  if constexpr (KSP == 2) {
+    // Both groups ran the same number of stages, so all eight waves met every
+    // barrier.  Group 1 hands its sums over through LDS (a 16-byte slot per
+    // lane and register quad) and is done; integer sums, so the result is the
+    // unsplit one exactly.
+    lds_barrier();   // every wave is done reading the stage buffers
+    int4* part = reinterpret_cast<int4*>(lds_all) + wave * (NT * MT * 4 * 64) + lane;
+    if (grp == 1) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            part[((j * MT + i) * 4 + q) * 64] = make_int4(acc[j][i][4 * q], acc[j][i][4 * q + 1],
+                                                          acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]);
+    }
+    lds_barrier();
+    if (grp == 1) {
+      lds_barrier();   // the epilogue's opening barrier
+      return;
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int4 o = part[((j * MT + i) * 4 + q) * 64];
+          acc[j][i][4 * q] += o.x;
+          acc[j][i][4 * q + 1] += o.y;
+          acc[j][i][4 * q + 2] += o.z;
+          acc[j][i][4 * q + 3] += o.w;
+        }
+  }
   if constexpr (OUT == 2) {
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
@@ -457,14 +505,58 @@ static int w8a8_col_group(long tiles_m, int tiles_n, long M, long K) {
   return best;
 }
 
-template <int MT, int OUT, bool PACKED>
+template <int MT, int OUT, bool PACKED, int KSP = 1>
 static void launch(const void* a, const void* b, const void* ws, const void* as, const void* bias,
                    const void* gamma, void* out, int M, int N, int K, hipStream_t st) {
   const int tiles_m = (M + 32 * MT - 1) / (32 * MT), tiles_n = (N + 255) / 256;
   const int gn = w8a8_col_group(tiles_m, tiles_n, M, K);
-  hipLaunchKernelGGL((w8a8_gemm_kernel<MT, OUT, PACKED>), dim3(tiles_m * tiles_n), dim3(256), 0, st,
+  hipLaunchKernelGGL((w8a8_gemm_kernel<MT, OUT, PACKED, KSP>), dim3(tiles_m * tiles_n), dim3(256 * KSP), 0, st,
                      (const int8_t*)a, (const int8_t*)b, (const uint16_t*)ws, (const uint16_t*)as,
                      (const uint16_t*)bias, (const uint16_t*)gamma, out, M, N, K, tiles_n, gn);
+}
+
+// The launch form, 10 MT + KSP, with the least estimated time.  The sums are
+// integers, so every form gives the same bits and the choice is free.
+// Estimate (us): workgroups fill 256 CUs, two a CU (K split: one of eight
+// waves); whole rounds and a last one of over 256 workgroups cost a pair each,
+// a last one of up to 256 a single; each is a + b * K / 1024.  The constants
+// are a least-squares fit to 36 shapes (M = 500 ... 10992, the four layers of
+// a VGGT block) x both weight layouts x the forms, 6-10 % off (rms); over them
+// the choice is 1 % off the best form and 7 % faster (geometric mean) than the
+// former rule, 128-row tiles where they number 256 and else 64-row ones:
+// packed 4122 x 4096 -> 1024 31.4 -> 25.0 us (96 rows, K split), 4122 x 1024
+// -> 4096 29.9 -> 26.0 (96 rows), 500 x 1024 -> 1024 7.0 -> 5.7 (32 rows);
+// stored 5496 x 4096 -> 1024 44.0 -> 38.2 (96 rows, K split).  The K split
+// pays from K = 2048 (at 1024 its hand-over costs what it saves); 32-row tiles
+// past half the chip only for short K on the packed layout (1374 x 4096 ->
+// 1024: 18.5 us packed and 33.3 stored, against 15.6 and 22.3 for 64 rows, K
+// split).  128 rows with K split spill; 32 rows with K split were nowhere better by
+// more than 4 %.
+static int w8a8_form(int64_t M, int64_t N, int64_t K, bool packed, bool ksplit) {
+  struct Form { int form; float s0, s1, p0, p1; };
+  static const Form forms[2][6] = {
+      {{41, 3.8f, 8.9f, 8.8f, 12.3f}, {31, 3.0f, 8.0f, 7.0f, 11.6f}, {21, 3.2f, 6.3f, 3.7f, 10.3f},
+       {11, 2.7f, 5.8f, 1.8f, 9.0f}, {32, 4.8f, 6.8f, 0.f, 0.f}, {22, 3.5f, 5.8f, 0.f, 0.f}},
+      {{41, 4.7f, 6.3f, 7.2f, 11.7f}, {31, 3.9f, 5.6f, 6.1f, 9.8f}, {21, 3.6f, 3.9f, 3.4f, 8.0f},
+       {11, 2.9f, 2.9f, 1.9f, 6.7f}, {32, 5.7f, 4.6f, 0.f, 0.f}, {22, 4.1f, 3.6f, 0.f, 0.f}}};
+  const int64_t tiles_n = (N + 255) / 256;
+  const float k = (float)K / 1024.0f;
+  int best = 0;
+  float best_t = 0.f;
+  for (const Form& f : forms[packed]) {
+    const int64_t bm = 32 * (f.form / 10), tiles = (M + bm - 1) / bm * tiles_n;
+    float t;
+    if (f.form % 10 == 2) {
+      if (!ksplit || K < 2048 || K % 128) continue;
+      t = (float)((tiles + 255) / 256) * (f.s0 + f.s1 * k);
+    } else {
+      if (f.form == 11 && tiles > 128 && (K >= 2048 || !packed)) continue;
+      const int64_t rem = tiles % 512;
+      t = (float)(tiles / 512 + (rem > 256)) * (f.p0 + f.p1 * k) + (rem > 0 && rem <= 256 ? f.s0 + f.s1 * k : 0.f);
+    }
+    if (!best || t < best_t) best = f.form, best_t = t;
+  }
+  return best;
 }
 
 // mode: 0 = fp16 out, 1 = fp16 out + bias, 2 = int32 accumulators,
@@ -489,24 +581,23 @@ static int w8a8_run(const void* a, const void* b, const void* ws, const void* as
   QV_CHECK_ARG((mode != 1 && mode != 3) || ((uintptr_t)bias % 8) == 0, "bias must be 8-byte aligned");
   QV_CHECK_ARG(mode != 3 || ((uintptr_t)gamma % 16) == 0, "gamma must be 16-byte aligned");
   hipStream_t st = (hipStream_t)stream;
-  const long big_tiles = (long)((M + 127) / 128) * ((N + 255) / 256);
-  const bool big = big_tiles >= 256;
   QV_CHECK_ARG(!packed || mode != 2, "the packed weight layout has no int32 output");
-#define QV_W8(MT, P)                                                                                \
-  switch (mode) {                                                                                   \
-    case 0: launch<MT, 0, P>(a, b, ws, as, bias, gamma, out, (int)M, (int)N, (int)K, st); break;    \
-    case 1: launch<MT, 1, P>(a, b, ws, as, bias, gamma, out, (int)M, (int)N, (int)K, st); break;    \
-    case 3: launch<MT, 3, P>(a, b, ws, as, bias, gamma, out, (int)M, (int)N, (int)K, st); break;    \
-    default:                                                                                        \
-      if constexpr (!P) launch<MT, 2, P>(a, b, ws, as, bias, gamma, out, (int)M, (int)N, (int)K, st); \
-      break;                                                                                        \
-  }
-  if (big) {
-    if (packed) { QV_W8(4, true) } else { QV_W8(4, false) }
-  } else {
-    if (packed) { QV_W8(2, true) } else { QV_W8(2, false) }
+#define QV_W8P(MT, OUT, P, KSP) launch<MT, OUT, P, KSP>(a, b, ws, as, bias, gamma, out, (int)M, (int)N, (int)K, st)
+#define QV_W8(MT, KSP)                                                                          \
+  if (mode == 0) packed ? QV_W8P(MT, 0, true, KSP) : QV_W8P(MT, 0, false, KSP);                 \
+  else if (mode == 1) packed ? QV_W8P(MT, 1, true, KSP) : QV_W8P(MT, 1, false, KSP);            \
+  else if (mode == 3) packed ? QV_W8P(MT, 3, true, KSP) : QV_W8P(MT, 3, false, KSP);            \
+  else if constexpr (KSP == 1) QV_W8P(MT, 2, false, 1);
+  switch (w8a8_form(M, N, K, packed, mode != 2)) {
+    case 41: QV_W8(4, 1) break;
+    case 31: QV_W8(3, 1) break;
+    case 21: QV_W8(2, 1) break;
+    case 11: QV_W8(1, 1) break;
+    case 32: QV_W8(3, 2) break;
+    default: QV_W8(2, 2) break;
   }
 #undef QV_W8
+#undef QV_W8P
   return check_launch("w8a8_gemm");
 }
 

@@ -545,3 +545,34 @@ def test_qknorm_rope2d_bit_exact(gpu, H, S):
     ref = R.qknorm_rope2d(x[:, :2], pos, c, s, qg, qb, kg, kb, 1e-6)
     assert np.array_equal(got[:, :2].view(np.int16), ref.view(np.int16))
     assert np.array_equal(got[:, 2], x[:, 2])
+
+
+@pytest.mark.parametrize("M,N,K", [(500, 1024, 1024), (33, 272, 192), (65, 1024, 4096), (1373, 4096, 1024), (97, 272, 4096),
+                                   (4122, 1024, 4096), (4037, 1040, 2176), (1374, 1024, 4096), (64, 16, 2304),
+                                   (2000, 1024, 2112), (5496, 3072, 1024)])
+def test_w8a8_launch_forms_bit_exact(gpu, M, N, K):
+    """The launch forms (32-, 64-, 96-, 128-row tiles; K split between two wave
+    groups, odd and even stage counts a group, K that cannot be split) on both
+    weight layouts and the residual form: the integer sums are exact (float64
+    products), so every form gives the epilogue's bits."""
+    from qvggt_amd import awq_inference_engine as E
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    a, w = (torch.randint(-128, 128, sh, generator=g, device=gpu, dtype=torch.int16).to(torch.int8) for sh in ((M, K), (N, K)))
+    ws, as_ = (torch.rand(n, generator=g, device=gpu).mul(1e-3).half() for n in (N, M))
+    bias, gamma = (torch.randn(N, generator=g, device=gpu).half() for _ in range(2))
+    res = torch.randn(M, N, generator=g, device=gpu).half()
+    acc = (a.double() @ w.double().t().contiguous()).float()
+    want = (acc * ws.float()[None] * as_.float()[:, None] + bias.float()[None]).half()
+    want_res = (res.float() + gamma.float()[None] * want.float()).half()
+    packed = E.w8a8_pack_weight(w)
+    out = [torch.full((M, N), float("nan"), device=gpu, dtype=torch.float16) for _ in range(2)]
+    E.w8a8_gemm_fuse_bias_forward_cuda(a, w, ws, as_, out[0], bias)
+    E.w8a8_gemm_packed(a, packed, N, ws, as_, out[1], bias=bias)
+    r = [res.clone(), res.clone()]
+    E.w8a8_linear_residual(a, w, ws, as_, bias, gamma, r[0])
+    E.w8a8_gemm_packed(a, packed, N, ws, as_, r[1], bias=bias, gamma=gamma)
+    for o in out:
+        assert torch.equal(o, want)
+    for o in r:
+        assert torch.equal(o, want_res)
+    assert torch.equal(E.w8a8_gemm_int32(a, w).float(), acc)
