@@ -322,6 +322,17 @@ int qv_attention_fwd(const void* q, const void* k, const void* v, void* out, int
                      int64_t k_token_stride, int64_t v_token_stride, int64_t out_token_stride,
                      float scale, void* stream);
 
+/* ---------------------------------------------------- fp16 linear
+ * No counterpart in the reference extension (the DINOv2 patch embed stays in
+ * floating point, qvggt/inference/loader.py:346, and its graph is in the
+ * external vggt-hf): out = epilogue(x w^T + bias), x (M, K), w (N, K), bias (N)
+ * fp16, fp32 sums, one rounding.  epilogue QV_EPI_BIAS or QV_EPI_BIAS_GELU;
+ * with gamma (N, QV_EPI_BIAS only) out += gamma * fp16(x w^T + bias) in place.
+ * K a multiple of 32, N of 16; x, w, out and gamma 16-byte, bias 8-byte aligned.
+ */
+int qv_f16_gemm(const void* x, const void* w, const void* bias, const void* gamma, void* out,
+                int64_t M, int64_t N, int64_t K, int epilogue, void* stream);
+
 /* ---------------------------------------------------- camera head
  * No counterparts in the reference extension: the camera head's graph is in
  * the external vggt-hf (qvggt/inference/loader.py:204-206 quantises its trunk

@@ -25,9 +25,9 @@ come from ``AggregatorConfig`` (a checkpoint's config.json); its defaults are
 the benchmark configuration's LayerNorm(1024, eps 1e-6) and 24 + 24 blocks.
 
 Every hot op runs on libqvggt_hip.so, the AA blocks' LayerScale residual
-updates included (fused into the proj / fc2 GEMMs); only the DINOv2 fp16
-linears and the patch projection (plain GEMMs: hipBLASLt through torch), its
-GELU and its LayerScale residual updates use torch.
+updates included (fused into the proj / fc2 GEMMs); only the DINOv2 qkv and
+fc2 linears and the patch projection (plain GEMMs: hipBLASLt through torch) and
+the fc2 residual update use torch.
 """
 from __future__ import annotations
 
@@ -264,8 +264,8 @@ def _linear(layer, x: torch.Tensor, epilogue: int, out: torch.Tensor) -> torch.T
     return y
 
 
-def _affine(ln: nn.LayerNorm):
-    """A norm's (weight, bias), read from its parameter table (see ``w4_buffers``)."""
+def _affine(ln: nn.Module):
+    """A norm's or linear's (weight, bias), read from its parameter table (see ``w4_buffers``)."""
     p = ln._parameters
     try:
         return p["weight"], p["bias"]
@@ -357,7 +357,8 @@ class AABlock(nn.Module):
 
 
 class DinoBlock(nn.Module):
-    """DINOv2 ViT-L block in fp16 (linears through hipBLASLt, LN/attention on our kernels)."""
+    """DINOv2 ViT-L block in fp16: LN, attention, proj (its LayerScale residual
+    fused) and fc1 (its GELU fused) on our kernels, qkv and fc2 through hipBLASLt."""
 
     def __init__(self, dev=None, eps: float = LN_EPS):
         super().__init__()
@@ -375,16 +376,17 @@ class DinoBlock(nn.Module):
     @torch.no_grad()
     def forward(self, x: torch.Tensor, ws: dict) -> torch.Tensor:
         M = x.shape[0]
-        h = E.layer_norm(x, self.norm1.weight, self.norm1.bias, self.eps, out=ws["h"])
-        qkv = torch.addmm(self.attn.qkv.bias, h, self.attn.qkv.weight.t(), out=ws["qkv"])
+        attn, mlp = self.attn, self.mlp
+        qkv_w, qkv_b = _affine(attn.qkv)
+        fc2_w, fc2_b = _affine(mlp.fc2)
+        h = E.layer_norm(x, *_affine(self.norm1), self.eps, out=ws["h"])
+        qkv = torch.addmm(qkv_b, h, qkv_w.t(), out=ws["qkv"])
         v3 = qkv.view(M, 3, HEADS, HEAD_DIM)
-        att = E.attention(v3[:, 0], v3[:, 1], v3[:, 2], TOKENS, out=ws["att"].view(M, HEADS, HEAD_DIM))
-        o = torch.addmm(self.attn.proj.bias, att.view(M, DIM), self.attn.proj.weight.t(), out=ws["o"])
-        x.addcmul_(o, self.ls1.gamma)
-        h = E.layer_norm(x, self.norm2.weight, self.norm2.bias, self.eps, out=ws["h"])
-        f = torch.addmm(self.mlp.fc1.bias, h, self.mlp.fc1.weight.t(), out=ws["f"])
-        f = F.gelu(f)
-        o = torch.addmm(self.mlp.fc2.bias, f, self.mlp.fc2.weight.t(), out=ws["o"])
+        att = E.attention(*v3.unbind(1), TOKENS, out=ws["att"].view(M, HEADS, HEAD_DIM))
+        E.f16_linear(att.view(M, DIM), *_affine(attn.proj), out=x, gamma=self.ls1.gamma)
+        h = E.layer_norm(x, *_affine(self.norm2), self.eps, out=ws["h"])
+        f = E.f16_linear(h, *_affine(mlp.fc1), QV_EPI_BIAS_GELU, out=ws["f"])
+        o = torch.addmm(fc2_b, f, fc2_w.t(), out=ws["o"])
         x.addcmul_(o, self.ls2.gamma)
         return x
 

@@ -760,6 +760,32 @@ def qknorm_rope2d(qkv: torch.Tensor, positions: torch.Tensor, cos_table: torch.T
     return qkv
 
 
+# ----------------------------------------------------------- fp16 linear
+def f16_linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, epilogue: int = _lib.QV_EPI_BIAS,
+               out: torch.Tensor | None = None, gamma: torch.Tensor | None = None) -> torch.Tensor:
+    """fp16 linear x (..., K) @ weight (N, K)^T + bias with its epilogue fused:
+    bias, bias + GELU (exact-erf), or, with ``gamma``, out += gamma * fp16(linear)
+    in place (``out`` the residual stream).  fp32 sums, one rounding."""
+    what = "f16_linear"
+    K = x.shape[-1]
+    M = x.numel() // K if K else 0
+    N = weight.shape[0]
+    for name, t, shape in (("x", x, x.shape), ("weight", weight, (N, K)), ("bias", bias, (N,))):
+        if t.dtype != torch.float16 or t.shape != shape:
+            _fail(f"{what}: {name} must be float16 {tuple(shape)}, got {tuple(t.shape)} {t.dtype}")
+    if gamma is not None and (gamma.dtype != torch.float16 or gamma.numel() != N or out is None):
+        _fail(f"{what}: the residual form needs out and gamma float16 ({N},)")
+    dev = _on_gpu(x, weight, bias, out, gamma, what=what)
+    if out is not None:
+        _check_out(out, M, N, x.dtype, what)
+    else:
+        out = x.new_empty((*x.shape[:-1], N))
+    x, w, b, g = _contig(x), _contig(weight), _contig(bias), _contig_opt(gamma)
+    with _device(dev):
+        _lib.call("qv_f16_gemm", _ptr(x), _ptr(w), _ptr(b), _ptr(g), _ptr(out), M, N, K, epilogue, _stream(dev))
+    return out
+
+
 # ----------------------------------------------------------- camera head
 def pose_attention(qkv: torch.Tensor, heads: int, scale: float) -> torch.Tensor:
     """Attention over the S pose tokens of a contiguous (S, 3*heads*128) fp16

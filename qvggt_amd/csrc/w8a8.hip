@@ -44,15 +44,27 @@ namespace qv {
 __device__ __forceinline__ int f8(int r) { return (r + (r >> 2)) & 3; }
 
 // OUT: 0 = fp16 (scaled), 1 = fp16 (scaled + bias), 2 = raw int32,
-// 3 = fp16 (scaled + bias) LayerScale-added to `out` in place
+// 3 = fp16 (scaled + bias) LayerScale-added to `out` in place, 4 = fp16
+// GELU(sum + bias) (F16 only)
+// F16: fp16 operands instead of int8 (qv_f16_gemm).  A 16-byte fragment is
+// then 8 halves of v_mfma_f32_32x32x16_f16 instead of 16 bytes of
+// v_mfma_i32_32x32x32_i8 -- the same bytes, LDS layout, pipeline and MFMA
+// cycles --, K counts bytes a row, the sums are fp32 and there are no scales.
 // KSP: 1, or 2 = K split between two 4-wave groups of one 8-wave workgroup
-template <int MT, int OUT, bool PACKED, int KSP>
+template <int MT, int OUT, bool PACKED, int KSP, bool F16 = false>
 __global__ __launch_bounds__(256 * KSP) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b,
                       const uint16_t* __restrict__ ws, const uint16_t* __restrict__ as,
                       const uint16_t* __restrict__ bias, const uint16_t* __restrict__ gamma,
                       void* __restrict__ out, int M, int N, int K, int tiles_n, int gn) {
-  constexpr bool BIAS = OUT == 1 || OUT == 3;
+  constexpr bool BIAS = OUT == 1 || OUT == 3 || OUT == 4;
+  using acc_t = std::conditional_t<F16, f32x16, i32x16>;
+  auto mfma = [](const uint4& bw, const uint4& av, const acc_t& c) __attribute__((always_inline)) {
+    if constexpr (F16)
+      return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, bw), __builtin_bit_cast(f16x8, av), c, 0, 0, 0);
+    else
+      return __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, bw), __builtin_bit_cast(i32x4, av), c, 0, 0, 0);
+  };
   constexpr int BM = 32 * MT, BN = 256, NT = 2;
   constexpr int A_BYTES = BM * 64, B_BYTES = PACKED ? 0 : BN * 64;
   constexpr int STAGE = A_BYTES + B_BYTES;
@@ -104,11 +116,11 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
 #pragma unroll
       for (int qd = 0; qd < 4; ++qd) {
         const int n = min(n0 + 64 * wave + 32 * j + 8 * qd + 4 * h, N - 4);
-        wsv[j][qd] = *reinterpret_cast<const uint2*>(ws + n);
+        if constexpr (!F16) wsv[j][qd] = *reinterpret_cast<const uint2*>(ws + n);
         if constexpr (BIAS) bsv[j][qd] = *reinterpret_cast<const uint2*>(bias + n);
       }
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
+    for (int i = 0; i < MT && !F16; ++i) {
       const int m = m0 + 32 * i + l32;
       asv[i] = as[m < M ? m : M - 1];
     }
@@ -146,7 +158,7 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
     }
   };
 
-  i32x16 acc[NT][MT];
+  acc_t acc[NT][MT];
 #pragma unroll
   for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -179,8 +191,7 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
       for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
-          acc[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, bw[j][s]),
-                                                            __builtin_bit_cast(i32x4, av[i]), acc[j][i], 0, 0, 0);
+          acc[j][i] = mfma(bw[j][s], av[i], acc[j][i]);
     };
     // One stage (LDS buffer st, weights bw), as in the LDS path below: step 0
     // issues the activation reads of step 1, then its MFMAs; step 1 those of
@@ -268,8 +279,7 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
       for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
-          acc[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, bw[j]),
-                                                            __builtin_bit_cast(i32x4, av[i]), acc[j][i], 0, 0, 0);
+          acc[j][i] = mfma(bw[j], av[i], acc[j][i]);
     };
     // One stage (buffer st).  On entry b0 / a0 hold its k-step 0 fragments.
     // Step 0 issues the reads of step 1, then its MFMAs; step 1 issues the
@@ -371,7 +381,9 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
     float am[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-      if constexpr (PREF) {
+      if constexpr (F16) {
+        am[i] = 1.f;
+      } else if constexpr (PREF) {
         am[i] = to_f32(asv[i], false);
       } else {
         const int m = m0 + 32 * i + l32;
@@ -385,8 +397,9 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
         const int nl = 32 * j + 8 * qd + 4 * h;
         const int n = min(n0 + 64 * wave + nl, N - 4);
         float wsn[4], bn[4] = {0.f, 0.f, 0.f, 0.f};
-        uint2 wv;
-        if constexpr (PREF) wv = wsv[j][qd];
+        uint2 wv = make_uint2(0, 0);
+        if constexpr (F16) {
+        } else if constexpr (PREF) wv = wsv[j][qd];
         else wv = *reinterpret_cast<const uint2*>(ws + n);
         wsn[0] = to_f32((uint16_t)(wv.x & 0xFFFF), false);
         wsn[1] = to_f32((uint16_t)(wv.x >> 16), false);
@@ -406,9 +419,10 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
           float r[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            float t = (float)acc[j][i][4 * qd + e] * wsn[e];
-            t = t * am[i];
+            float t = (float)acc[j][i][4 * qd + e];
+            if constexpr (!F16) t = t * wsn[e] * am[i];
             if constexpr (BIAS) t = t + bn[e];
+            if constexpr (OUT == 4) t = gelu_erf(t);
             // keep the fp32 rounding of t: without this the backend fuses the last
             // multiply and the fp16 conversion into one v_fma_mixlo_f16 (one rounding)
             asm volatile("" : "+v"(t));
@@ -505,12 +519,12 @@ static int w8a8_col_group(long tiles_m, int tiles_n, long M, long K) {
   return best;
 }
 
-template <int MT, int OUT, bool PACKED, int KSP = 1>
+template <int MT, int OUT, bool PACKED, int KSP = 1, bool F16 = false>
 static void launch(const void* a, const void* b, const void* ws, const void* as, const void* bias,
                    const void* gamma, void* out, int M, int N, int K, hipStream_t st) {
   const int tiles_m = (M + 32 * MT - 1) / (32 * MT), tiles_n = (N + 255) / 256;
   const int gn = w8a8_col_group(tiles_m, tiles_n, M, K);
-  hipLaunchKernelGGL((w8a8_gemm_kernel<MT, OUT, PACKED, KSP>), dim3(tiles_m * tiles_n), dim3(256 * KSP), 0, st,
+  hipLaunchKernelGGL((w8a8_gemm_kernel<MT, OUT, PACKED, KSP, F16>), dim3(tiles_m * tiles_n), dim3(256 * KSP), 0, st,
                      (const int8_t*)a, (const int8_t*)b, (const uint16_t*)ws, (const uint16_t*)as,
                      (const uint16_t*)bias, (const uint16_t*)gamma, out, M, N, K, tiles_n, gn);
 }
@@ -602,6 +616,43 @@ static int w8a8_run(const void* a, const void* b, const void* ws, const void* as
 }
 
 }  // namespace qv
+
+// fp16 linear on the int8 kernel's stored-layout form (tile heights by the same
+// estimate, K in bytes a row).  Bound by LDS bandwidth: both operands pass
+// through it, 6 KB of fragments per 8 MFMAs a wave plus the copies, ~140 bytes
+// a clock at full MFMA rate against 128.  What it gains over the library's
+// product is the fused epilogue: bias + GELU 1024 -> 4096 in 64.5 us against
+// 63 + 17 at M = 5496 (22 / 29 at 1374, 100 / 112 at 8244, 220 / 260 at 21984),
+// bias + residual 1024 -> 1024 in 25.2 against 18.5 + 9.5.  Without one (qkv),
+// or at K = 4096, the library's product is faster (43 / 52 us, 49 / 77).
+extern "C" int qv_f16_gemm(const void* x, const void* w, const void* bias, const void* gamma, void* out, int64_t M,
+                           int64_t N, int64_t K, int epilogue, void* stream) {
+  using namespace qv;
+  QV_CHECK_ARG(M >= 0 && N > 0 && K > 0, "bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
+  QV_CHECK_ARG(K % 32 == 0 && N % 16 == 0, "K=%lld must be a multiple of 32 and N=%lld of 16", (long long)K, (long long)N);
+  QV_CHECK_ARG(M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX / 2, "shape too large");
+  QV_CHECK_ARG((uint64_t)N * K * 2 < (1ull << 32) && (uint64_t)256 * K < (1ull << 31),
+               "weight too large for 32-bit offsets");
+  QV_CHECK_ARG(epilogue == QV_EPI_BIAS || epilogue == QV_EPI_BIAS_GELU, "unsupported epilogue %d", epilogue);
+  QV_CHECK_ARG(!gamma || epilogue == QV_EPI_BIAS, "the residual form takes the bias epilogue");
+  if (M == 0) return QV_OK;
+  QV_CHECK_ARG(x && w && bias && out, "null pointer argument");
+  QV_CHECK_ARG((((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)gamma) % 16) == 0 && ((uintptr_t)bias % 8) == 0,
+               "x, w, gamma and out must be 16-byte and bias 8-byte aligned");
+  hipStream_t st = (hipStream_t)stream;
+  const int K2 = (int)K * 2;   // bytes a row
+#define QV_F16P(MT, OUT) launch<MT, OUT, false, 1, true>(x, w, nullptr, nullptr, bias, gamma, out, (int)M, (int)N, K2, st)
+#define QV_F16(MT) gamma ? QV_F16P(MT, 3) : epilogue == QV_EPI_BIAS ? QV_F16P(MT, 1) : QV_F16P(MT, 4);
+  switch (w8a8_form(M, N, K2, false, false)) {
+    case 41: QV_F16(4) break;
+    case 31: QV_F16(3) break;
+    case 21: QV_F16(2) break;
+    default: QV_F16(1) break;
+  }
+#undef QV_F16
+#undef QV_F16P
+  return check_launch("f16_gemm");
+}
 
 extern "C" int qv_w8a8_gemm(const int8_t* a, const int8_t* b, const void* wscales, const void* ascales,
                             const void* bias, void* out, int64_t M, int64_t N, int64_t K, void* stream) {

@@ -576,3 +576,34 @@ def test_w8a8_launch_forms_bit_exact(gpu, M, N, K):
     for o in r:
         assert torch.equal(o, want_res)
     assert torch.equal(E.w8a8_gemm_int32(a, w).float(), acc)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (33, 272, 96), (65, 1024, 1024), (97, 1040, 160), (1374, 4096, 1024),
+                                   (4122, 1024, 1024), (5497, 4096, 1024)])
+@pytest.mark.parametrize("mode", ["bias", "gelu", "residual"])
+def test_f16_linear(gpu, M, N, K, mode):
+    """fp16 linear on the int8 kernel's pipeline, all tile heights and their
+    remainders, one to sixteen times two stages, against float64.  Bounds: one
+    fp16 rounding (2^-11 relative; the residual form rounds the linear and the
+    sum; GELU's polynomial is within one more step, 2^-10), plus the fp32 sum's
+    K * 2^-24 of the absolute terms."""
+    from qvggt_amd import awq_inference_engine as E
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    x, w, b, ga, r = (torch.randn(sh, generator=g, device=gpu).mul(sc).half() for sh, sc in
+                      (((M, K), 1.0), ((N, K), K ** -0.5), ((N,), 0.5), ((N,), 0.5), ((M, N), 1.0)))
+    lin = x.double() @ w.double().t().contiguous() + b.double()
+    terms = (x.double().abs() @ w.double().abs().t().contiguous()) * (K * 2.0 ** -24)
+    if mode == "residual":
+        got = E.f16_linear(x, w, b, out=r.clone(), gamma=ga)
+        ref = r.double() + ga.double() * lin
+        bound = ref.abs() * 2.0 ** -11 + ga.double().abs() * (lin.abs() * 2.0 ** -11 + terms)
+    elif mode == "gelu":
+        got, ref = E.f16_linear(x, w, b, 2), torch.nn.functional.gelu(lin)
+        bound = ref.abs() * (2.0 ** -11 + 2.0 ** -10) + terms * 1.2
+    else:
+        got, ref, bound = E.f16_linear(x, w, b), lin, lin.abs() * 2.0 ** -11 + terms
+    assert ((got.double() - ref).abs() <= bound + 2.0 ** -24).all()
+    strided = torch.zeros(M, K + 8, device=gpu, dtype=torch.float16)
+    strided[:, :K] = x
+    if mode == "bias":
+        assert torch.equal(E.f16_linear(strided[:, :K], w, b), got)
