@@ -216,114 +216,136 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(QB =
 
   // one 64-key compute tile: keys key0.., K / V rows at kb_lds / vb
   auto ctile = [&](int key0, const uint8_t* kb_lds, const uint8_t* vb, bool mask) __attribute__((always_inline)) {
-    {
-      // ---- S^T = K Q^T for the 64 keys of the tile, both query blocks (raw dot products)
-      f32x16 sc[QB][2];   // [query block][key block]
-  #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
+    f32x16 sc[QB][2];   // [query block][key block]
+    uint4 kf[2][4], vfr[2][4], pf[QB][4];
+    float t = 0.f;
+    auto qk1 = [&](int qb, int kb, int st) __attribute__((always_inline)) {
+      sc[qb][kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, kf[kb][st]),
+                                                          __builtin_bit_cast(f16x8, qf[qb][st]),
+                                                          st == 0 ? f32x16{} - base[qb] : sc[qb][kb], 0, 0, 0);
+    };
+    auto pv1 = [&](int qb, int db, int st) __attribute__((always_inline)) {
+      o[qb][db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, vfr[db][st]),
+                                                         __builtin_bit_cast(f16x8, pf[qb][st]), o[qb][db], 0, 0, 0);
+    };
+    auto read_v = [&](int db, int st) __attribute__((always_inline)) {
+      const int dim = 32 * db + tr_dim;
+      uint2 vv[2];
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        const int key = 16 * st + 8 * r + tr_key;
+        vv[r] = lds_read_tr16(vb + key * 128 + (((dim >> 3) ^ fv(key)) * 16) + ((dim >> 2) & 1) * 8);
+      }
+      vfr[db][st] = make_uint4(vv[0].x, vv[0].y, vv[1].x, vv[1].y);
+    };
+    auto mask_keys = [&](int qb) __attribute__((always_inline)) {
+      const int kh = key0 + 4 * h;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (kh + 32 * kb + 8 * (r >> 2) + (r & 3) >= L) sc[qb][kb][r] = -INFINITY;
+    };
+    // word w (0..15) of a query block's packed P: its scores 2 w, 2 w + 1
+    auto p_word = [&](int qb, int w, bool shift, float off) __attribute__((always_inline)) {
+      const float s0 = sc[qb][w >> 3][2 * (w & 7)], s1 = sc[qb][w >> 3][2 * (w & 7) + 1];
+      const float p0 = __builtin_amdgcn_exp2f(shift ? s0 + off : s0);
+      const float p1 = __builtin_amdgcn_exp2f(shift ? s1 + off : s1);
+      const f16x2 ph = {(_Float16)p0, (_Float16)p1};
+      t += p0;
+      t += p1;
+      return __builtin_bit_cast(uint32_t, ph);
+    };
+    auto set_p = [&](int qb, const uint32_t (&pw)[16]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int st = 0; st < 4; ++st) pf[qb][st] = make_uint4(pw[4 * st], pw[4 * st + 1], pw[4 * st + 2], pw[4 * st + 3]);
+    };
+    // P = 2^S' = 2^(S - m_use) of a query block in fp16 against the current
+    // reference, with the tile's partial row sum t (of the fp32 values).  The
+    // tile maximum is only needed when some P could exceed 2^RESCALE_SLACK,
+    // and every such P makes t exceed it too (P >= 0), so the maximum is
+    // computed only for waves where some lane's t does, and on the first tile
+    // (no reference yet).
+    // QB = 2: slot(i) comes before each of 8 fenced groups of four exp2, so
+    // that block 1's QK MFMAs run beside block 0's exp2 and block 0's PV MFMAs
+    // beside block 1's (left to the compiler the MFMAs clustered: 10992 tokens
+    // 488 -> 481 us, 8 x 1374 75.2 -> 73.0, 43968 7.12 -> 7.07 ms, the same
+    // bits; at QB = 1 fencing cost 5 % at 1 x 1374 and is left out).
+    auto softmax = [&](int qb, auto&& slot) __attribute__((always_inline)) {
+      if (mask) mask_keys(qb);
+      uint32_t pw[16];
+      t = 0.f;
+      if constexpr (QB == 2) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        slot(i);
+        pw[2 * i] = p_word(qb, 2 * i, false, 0.f);
+        pw[2 * i + 1] = p_word(qb, 2 * i + 1, false, 0.f);
+        if constexpr (QB == 2) __builtin_amdgcn_sched_barrier(0);
+      }
+      if (__builtin_amdgcn_ballot_w64(!(t <= P_SUM_LIMIT) || m_use[qb] == -INFINITY)) {
+        // ---- tile maximum of this query (both lane halves hold 32 keys each)
+        float mx = sc[qb][0][0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[qb][0][r]);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[qb][1][r]);
+        mx = half_max(mx) + base[qb];
+        const bool need = mx > m_use[qb] + RESCALE_SLACK;
+        if (__builtin_amdgcn_ballot_w64(need)) {
+          const float m_new = need ? mx : m_use[qb];
+          const float alpha = __builtin_amdgcn_exp2f(m_use[qb] - m_new);  // 0 on the first tile, 1 if !need
+          m_use[qb] = m_new;
+          l_run[qb] *= alpha;
+#pragma unroll
+          for (int db = 0; db < 2; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[qb][db][r] *= alpha;
+          t = 0.f;
+          const float off = base[qb] - m_new;
+#pragma unroll
+          for (int w = 0; w < 16; ++w) pw[w] = p_word(qb, w, true, off);
+        }
+        base[qb] = m_use[qb];
+      }
+      l_run[qb] += t;
+      set_p(qb, pw);
+    };
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
         const int row = 32 * kb + l32;
-  #pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          const int c = 2 * st + h;
-          const uint4 kf = *reinterpret_cast<const uint4*>(kb_lds + row * 128 + ((c ^ fk(row)) * 16));
-  #pragma unroll
-          for (int qb = 0; qb < QB; ++qb)
-            sc[qb][kb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                __builtin_bit_cast(f16x8, kf), __builtin_bit_cast(f16x8, qf[qb][st]),
-                st == 0 ? f32x16{} - base[qb] : sc[qb][kb], 0, 0, 0);
-        }
+        kf[kb][st] = *reinterpret_cast<const uint4*>(kb_lds + row * 128 + (((2 * st + h) ^ fk(row)) * 16));
       }
-      // ---- V^T fragments of this tile, read before the softmax so their LDS
-      // latency hides behind it (the PV MFMAs below consume them)
-      uint4 vfr[2][4];
-  #pragma unroll
-      for (int db = 0; db < 2; ++db) {
-        const int dim = 32 * db + tr_dim;
-  #pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          uint2 vv[2];
-  #pragma unroll
-          for (int r = 0; r < 2; ++r) {
-            const int key = 16 * st + 8 * r + tr_key;
-            vv[r] = lds_read_tr16(vb + key * 128 + (((dim >> 3) ^ fv(key)) * 16) + ((dim >> 2) & 1) * 8);
-          }
-          vfr[db][st] = make_uint4(vv[0].x, vv[0].y, vv[1].x, vv[1].y);
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) qk1(0, kb, st);
+    if constexpr (QB == 2) {
+      softmax(0, [&](int i) __attribute__((always_inline)) {
+        qk1(1, i & 1, i >> 1);
+        if (i >= 4) {   // V^T fragments, as the K fragments' registers fall free
+          read_v(0, i - 4);
+          read_v(1, i - 4);
         }
+      });
+      softmax(1, [&](int i) __attribute__((always_inline)) { pv1(0, i & 1, i >> 1); });
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int db = 0; db < 2; ++db) pv1(1, db, st);
+    } else {
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        read_v(0, st);
+        read_v(1, st);
       }
-      uint4 pf[QB][4];
-  #pragma unroll
-      for (int qb = 0; qb < QB; ++qb) {
-        if (mask) {
-          const int kh = key0 + 4 * h;
-  #pragma unroll
-          for (int kb = 0; kb < 2; ++kb)
-  #pragma unroll
-            for (int r = 0; r < 16; ++r)
-              if (kh + 32 * kb + 8 * (r >> 2) + (r & 3) >= L) sc[qb][kb][r] = -INFINITY;
-        }
-        // ---- P = 2^S' = 2^(S - m_use) in fp16 against the current reference,
-        // with this tile's partial row sum t (of the fp32 values).  The
-        // tile maximum is only needed when some P could exceed 2^RESCALE_SLACK,
-        // and every such P makes t exceed it too (P >= 0), so the maximum is
-        // computed only for waves where some lane's t does, and on the first
-        // tile (no reference yet).
-        float t = 0.f;
-        auto make_p = [&](bool shift, float off) {
-  #pragma unroll
-          for (int kb = 0; kb < 2; ++kb)
-  #pragma unroll
-            for (int pp = 0; pp < 2; ++pp) {
-              uint32_t w[4];
-  #pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                const float s0 = sc[qb][kb][8 * pp + 2 * e], s1 = sc[qb][kb][8 * pp + 2 * e + 1];
-                const float p0 = __builtin_amdgcn_exp2f(shift ? s0 + off : s0);
-                const float p1 = __builtin_amdgcn_exp2f(shift ? s1 + off : s1);
-                const f16x2 ph = {(_Float16)p0, (_Float16)p1};
-                t += p0;
-                t += p1;
-                w[e] = __builtin_bit_cast(uint32_t, ph);
-              }
-              pf[qb][2 * kb + pp] = make_uint4(w[0], w[1], w[2], w[3]);
-            }
-        };
-        make_p(false, 0.f);
-        if (__builtin_amdgcn_ballot_w64(!(t <= P_SUM_LIMIT) || m_use[qb] == -INFINITY)) {
-          // ---- tile maximum of this query (both lane halves hold 32 keys each)
-          float mx = sc[qb][0][0];
-  #pragma unroll
-          for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[qb][0][r]);
-  #pragma unroll
-          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[qb][1][r]);
-          mx = half_max(mx) + base[qb];
-          // ---- lazy rescale: the reference moves when the tile maximum exceeds
-          // it by more than the slack; then P is recomputed against it
-          const bool need = mx > m_use[qb] + RESCALE_SLACK;
-          if (__builtin_amdgcn_ballot_w64(need)) {
-            const float m_new = need ? mx : m_use[qb];
-            const float alpha = __builtin_amdgcn_exp2f(m_use[qb] - m_new);  // 0 on the first tile, 1 if !need
-            m_use[qb] = m_new;
-            l_run[qb] *= alpha;
-  #pragma unroll
-            for (int db = 0; db < 2; ++db)
-  #pragma unroll
-              for (int r = 0; r < 16; ++r) o[qb][db][r] *= alpha;
-            t = 0.f;
-            make_p(true, base[qb] - m_new);
-          }
-          base[qb] = m_use[qb];
-        }
-        l_run[qb] += t;
-        // ---- O^T += V^T P^T for this query block (each V^T fragment feeds
-        // both blocks), issued before the next block's softmax so these
-        // MFMAs run under its VALU work
-  #pragma unroll
-        for (int db = 0; db < 2; ++db)
-  #pragma unroll
-          for (int st = 0; st < 4; ++st)
-            o[qb][db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, vfr[db][st]),
-                                                              __builtin_bit_cast(f16x8, pf[qb][st]), o[qb][db], 0, 0, 0);
-      }
+      softmax(0, [](int) __attribute__((always_inline)) {});
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int db = 0; db < 2; ++db) pv1(0, db, st);
     }
   };
   auto tile = [&](int j, bool last) {
