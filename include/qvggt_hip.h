@@ -362,6 +362,26 @@ int qv_adaln_modulate(const void* mod, const void* adaln, const void* pose, void
 int qv_pose_update(const void* delta, float* pred, float* act, void* half, int64_t S, int64_t cols,
                    int64_t n_linear, int first, void* stream);
 
+/*
+ * The head's fp16 linears with what follows them, on few tokens (weights read
+ * once per 16): w rows contiguous fp16, fp32 sums, 16-byte aligned x and w, K
+ * a multiple of 32.
+ * qv_pose_embed: out (S, N) = silu(src w^T + bias), src (S, C <= 16) rows
+ * src_stride apart (0 repeats one row).  qv_pose_linear_gelu: out = gelu(x w^T
+ * + bias).  qv_pose_modulate: w (3 D, K), bias (3 D) give shift, scale and
+ * gate; x = gate * (adaln * (1 + scale) + shift) + pose.  qv_pose_delta:
+ * qv_pose_update with delta = x w^T + bias in fp32.
+ */
+int qv_pose_embed(const void* src, int64_t src_stride, const void* w, const void* bias, void* out,
+                  int64_t S, int64_t N, int64_t C, void* stream);
+int qv_pose_linear_gelu(const void* x, const void* w, const void* bias, void* out, int64_t S,
+                        int64_t N, int64_t K, void* stream);
+int qv_pose_modulate(const void* e, const void* w, const void* bias, const void* adaln,
+                     const void* pose, void* x, int64_t S, int64_t D, int64_t K, void* stream);
+int qv_pose_delta(const void* x, const void* w, const void* bias, float* pred, float* act,
+                  void* half, int64_t S, int64_t cols, int64_t K, int64_t n_linear, int first,
+                  void* stream);
+
 #ifdef __cplusplus
 }
 #endif

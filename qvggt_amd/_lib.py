@@ -54,6 +54,10 @@ SIGNATURES: dict[str, list] = {
     "qv_qknorm_rope2d": [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _f32, _i64, _i64, _i64, _vp],
     "qv_f16_gemm": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "qv_pose_attention": [_vp, _vp, _i64, _i64, _i64, _f32, _vp],
+    "qv_pose_embed": [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
+    "qv_pose_linear_gelu": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
+    "qv_pose_modulate": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
+    "qv_pose_delta": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp],
     "qv_adaln_modulate": [_vp, _vp, _vp, _vp, _i64, _i64, _vp],
     "qv_pose_update": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "qv_attention_fwd": [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _vp],

@@ -830,3 +830,76 @@ def pose_update(delta: torch.Tensor, pred: torch.Tensor, first: bool, n_linear: 
         _lib.call("qv_pose_update", _ptr(d), _ptr(pred), _ptr(act), _ptr(half), pred.shape[0], pred.shape[1], n_linear,
                   1 if first else 0, _stream(dev))
     return act, half
+
+
+def _pose_linear_args(x, weight, bias, N, what, *others):
+    """Checks of the camera head's fp16 linears: x (S, K), weight (N, K), bias
+    (N,); returns the device index and contiguous x, weight, bias."""
+    if x.dim() != 2:
+        _fail(f"{what}: x must be 2-D, got {tuple(x.shape)}")
+    for name, t, shape in (("x", x, tuple(x.shape)), ("weight", weight, (N, x.shape[1])), ("bias", bias, (N,))):
+        if t.dtype != torch.float16 or tuple(t.shape) != shape:
+            _fail(f"{what}: {name} must be float16 {shape}, got {tuple(t.shape)} {t.dtype}")
+    dev = _on_gpu(x, weight, bias, *others, what=what)
+    return dev, _contig(x), _contig(weight), _contig(bias)
+
+
+def pose_embed(src: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
+    """silu(src @ weight^T + bias): src (S, C <= 16) fp16, its rows contiguous
+    (or one row expanded), weight (N, C)."""
+    what = "pose_embed"
+    S, N = src.shape[0], weight.shape[0]
+    if src.dim() != 2 or (src.shape[1] > 1 and src.stride(1) != 1) or src.stride(0) < 0:
+        _fail(f"{what}: src must be 2-D with unit column stride")
+    for name, t, shape in (("src", src, tuple(src.shape)), ("weight", weight, (N, src.shape[1])), ("bias", bias, (N,))):
+        if t.dtype != torch.float16 or tuple(t.shape) != shape:
+            _fail(f"{what}: {name} must be float16 {shape}, got {tuple(t.shape)} {t.dtype}")
+    dev = _on_gpu(src, weight, bias, what=what)
+    w, b = _contig(weight), _contig(bias)
+    out = src.new_empty((S, N))
+    with _device(dev):
+        _lib.call("qv_pose_embed", _ptr(src), src.stride(0), _ptr(w), _ptr(b), _ptr(out), S, N, src.shape[1], _stream(dev))
+    return out
+
+
+def pose_linear_gelu(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
+    """gelu(x @ weight^T + bias) on few tokens, fp16, one rounding."""
+    N = weight.shape[0]
+    dev, x, w, b = _pose_linear_args(x, weight, bias, N, "pose_linear_gelu")
+    out = x.new_empty((x.shape[0], N))
+    with _device(dev):
+        _lib.call("qv_pose_linear_gelu", _ptr(x), _ptr(w), _ptr(b), _ptr(out), x.shape[0], N, x.shape[1], _stream(dev))
+    return out
+
+
+def pose_modulate(e: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, adaln: torch.Tensor,
+                  pose: torch.Tensor) -> torch.Tensor:
+    """``adaln_modulate`` with mod = e @ weight^T + bias kept in fp32; weight (3D, K)."""
+    what = "pose_modulate"
+    S, D = adaln.shape
+    dev, e, w, b = _pose_linear_args(e, weight, bias, 3 * D, what, adaln, pose)
+    for name, t in (("adaln", adaln), ("pose", pose)):
+        if t.dtype != torch.float16 or tuple(t.shape) != (e.shape[0], D):
+            _fail(f"{what}: {name} must be float16 ({e.shape[0]}, {D})")
+    adaln, pose = _contig(adaln), _contig(pose)
+    x = torch.empty_like(pose)
+    with _device(dev):
+        _lib.call("qv_pose_modulate", _ptr(e), _ptr(w), _ptr(b), _ptr(adaln), _ptr(pose), _ptr(x), S, D, e.shape[1],
+                  _stream(dev))
+    return x
+
+
+def pose_delta(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, pred: torch.Tensor, first: bool,
+               n_linear: int):
+    """``pose_update`` with delta = x @ weight^T + bias kept in fp32."""
+    what = "pose_delta"
+    cols = weight.shape[0]
+    dev, x, w, b = _pose_linear_args(x, weight, bias, cols, what, pred)
+    _need(pred, torch.float32, what, "pred")
+    if tuple(pred.shape) != (x.shape[0], cols):
+        _fail(f"{what}: pred must be ({x.shape[0]}, {cols})")
+    act, half = torch.empty_like(pred), torch.empty_like(pred, dtype=torch.float16)
+    with _device(dev):
+        _lib.call("qv_pose_delta", _ptr(x), _ptr(w), _ptr(b), _ptr(pred), _ptr(act), _ptr(half), x.shape[0], cols,
+                  x.shape[1], n_linear, 1 if first else 0, _stream(dev))
+    return act, half

@@ -23,7 +23,9 @@ the trunk blocks, 1e-6 for ``adaln_norm``.
 Per frame there is one pose token, so the trunk linears run at M = S: every
 S <= 64 runs on the skinny-M MFMA kernel (through the GEMV entry for
 S <= 16 and the GEMM entry above).  Attention over the S tokens (head_dim
-128, fp32; up to 256 frames), the adaLN modulation and the pose update are one kernel each.
+128, fp32; up to 256 frames) is one kernel; up to 64 frames the head's own fp16
+linears run with what surrounds them (SiLU, the adaLN modulation, GELU, the
+pose update) in four.
 ``GraphedCameraHead`` records the whole forward as one HIP graph.  The CICT token
 QVGGT's loader can attach (loader.py:224-246) has no public definition and is
 not modelled.
@@ -50,6 +52,30 @@ ADALN_EPS = 1e-6
 # fp32 batched products of torch are as fast or faster (256 frames: 24 us
 # against 96; 512: 74 / 63; 1024: 262 / 150).
 POSE_ATTENTION_MAX = 256
+
+
+# Frames up to which the head's own fp16 linears run on the few-token kernels,
+# which read the weights once per 16 tokens (beyond, the library's products).
+POSE_LINEAR_MAX = 64
+
+
+def _plain(*modules) -> bool:
+    """Whether calling the modules does nothing but their own forward: no hooks
+    on them or on all modules, the linears plain fp16 ones with a bias."""
+    g = nn.modules.module
+    if g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks:
+        return False
+    for m in modules:
+        if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__:
+            return False
+        if isinstance(m, nn.Linear):
+            p = m._parameters
+            if (type(m) is not nn.Linear or p.get("weight") is None or p.get("bias") is None
+                    or p["weight"].dtype != torch.float16 or p["bias"].dtype != torch.float16):
+                return False
+        elif type(m) not in (nn.Sequential, nn.SiLU):
+            return False
+    return True
 
 
 class TrunkBlock(nn.Module):
@@ -166,20 +192,27 @@ class CameraHead(nn.Module):
         src = self.empty_pose_tokens.view(1, POSE_DIM).expand(S, POSE_DIM)
         pred = torch.empty(S, POSE_DIM, dtype=torch.float32, device=tokens.device)
         outs = []
+        embed, modulation, fc1, fc2 = self.embed_pose, self.poseLN_modulation, self.pose_branch.fc1, self.pose_branch.fc2
+        fused = S <= POSE_LINEAR_MAX and _plain(embed, modulation, *modulation, fc1, fc2) and not torch.is_autocast_enabled()
         for i in range(num_iterations):
-            x = E.adaln_modulate(self.poseLN_modulation(self.embed_pose(src)), adaln, pose)
+            if fused:
+                x = E.pose_modulate(E.pose_embed(src, *_affine(embed)), *_affine(modulation[1]), adaln, pose)
+            else:
+                x = E.adaln_modulate(modulation(embed(src)), adaln, pose)
             for blk in self.trunk:
                 blk(x)
-            h = E.layer_norm(x, self.trunk_norm.weight, self.trunk_norm.bias, LN_EPS)
-            delta = self.pose_branch.fc2(F.gelu(self.pose_branch.fc1(h)))
-            act, src = E.pose_update(delta, pred, i == 0, 7)
+            h = E.layer_norm(x, *_affine(self.trunk_norm), LN_EPS)
+            if fused:
+                act, src = E.pose_delta(E.pose_linear_gelu(h, *_affine(fc1)), *_affine(fc2), pred, i == 0, 7)
+            else:
+                act, src = E.pose_update(fc2(F.gelu(fc1(h))), pred, i == 0, 7)
             outs.append(act)
         return outs
 
 
 class GraphedCameraHead:
     """``CameraHead.forward`` for a fixed frame count S, recorded once as a HIP
-    graph and replayed: the head is ~150 small launches per call (4 iterations
+    graph and replayed: the head is ~140 small launches per call (4 iterations
     x 4 trunk blocks of LayerNorm, four W4 linears at M = S, attention and
     residual updates), so replay removes the host launch cost that otherwise
     dominates at small S.  ``__call__(tokens)`` copies ``tokens`` (S, 2048)

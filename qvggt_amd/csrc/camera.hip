@@ -7,6 +7,8 @@
 // arithmetic; what pays is doing in one launch what the chain did in several.
 // As torch ops the attention took 9 launches, the modulation 7, the pose update
 // 5: the eager head at 8 frames went from 4.0 to 2.3 ms, ~400 launches to ~150.
+#include <type_traits>
+
 #include "common.h"
 
 namespace qv {
@@ -165,7 +167,171 @@ __global__ __launch_bounds__(256) void pose_update_kernel(const uint16_t* __rest
   half[i] = from_f32<false>(p);
 }
 
+// ------------------------------------------------ fp16 linears of the head
+// silu(src w^T + b) for src (S, C <= 16) and w (N, C): the embedded pose.
+// One output a thread.
+__global__ __launch_bounds__(256) void pose_embed_kernel(const uint16_t* __restrict__ src, long src_stride,
+                                                         const uint16_t* __restrict__ w,
+                                                         const uint16_t* __restrict__ b, uint16_t* __restrict__ out,
+                                                         int S, int N, int C) {
+  const int n = blockIdx.x * 256 + threadIdx.x, s = blockIdx.y;
+  if (n >= N) return;
+  float e = to_f32(b[n], false);
+  for (int c = 0; c < C; ++c)
+    e = __builtin_fmaf(to_f32(src[s * src_stride + c], false), to_f32(w[(long)n * C + c], false), e);
+  out[(long)s * N + n] = from_f32<false>(e / (1.0f + expf(-e)));
+}
+
+// x w^T of up to 16 tokens a workgroup row (blockIdx.y) and 16 channels of each
+// of PARTS weight blocks (N rows apart): 8 waves split K in steps of 32, the
+// weights are the A operand and the tokens the B operand of
+// v_mfma_f32_16x16x32_f16, partial sums meet in LDS and wave 0 finishes:
+//  MODE 0: out = gelu(sum + b)
+//  MODE 1: PARTS = 3 (shift, scale, gate): out = gate * (adaln * (1 + scale)
+//          + shift) + pose
+//  MODE 2: the pose update of pose_update_kernel with delta = sum + b
+// Bound by latency and the weight stream (25 MB at 2048 -> 3 x 2048).  As
+// library products with torch's passes between them an iteration's four
+// linears took ~35 us of GPU time and ~25 us of host time each.
+struct PoseTail {
+  const uint16_t *adaln, *pose;
+  float *pred, *act;
+  uint16_t* half;
+  int n_linear, first;
+};
+
+template <int MODE, int PARTS>
+__global__ __launch_bounds__(512) void pose_linear_kernel(const uint16_t* __restrict__ x,
+                                                          const uint16_t* __restrict__ w,
+                                                          const uint16_t* __restrict__ bias,
+                                                          uint16_t* __restrict__ out, int S, int N, int K, PoseTail tail) {
+  constexpr int W = 8;
+  __shared__ float4 part[W][PARTS][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane & 15, g = lane >> 4;
+  const int n_a = blockIdx.x * 16 + c, t_b = blockIdx.y * 16 + c;
+  // rows past N and tokens past S repeat the last one; their results are not stored
+  const uint16_t* wp = w + (long)(n_a < N ? n_a : N - 1) * K + 8 * g;
+  const uint16_t* xp = x + (long)(t_b < S ? t_b : S - 1) * K + 8 * g;
+  f32x4 acc[PARTS];
+#pragma unroll
+  for (int p = 0; p < PARTS; ++p) acc[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // U steps' loads are issued together, then their products
+  auto steps = [&](int k, auto uc) __attribute__((always_inline)) {
+    constexpr int U = decltype(uc)::value;
+    uint4 b[U], a[U][PARTS];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      b[u] = *reinterpret_cast<const uint4*>(xp + k + 32 * W * u);
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p) a[u][p] = *reinterpret_cast<const uint4*>(wp + (long)p * N * K + k + 32 * W * u);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p)
+        acc[p] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a[u][p]),
+                                                        __builtin_bit_cast(f16x8, b[u]), acc[p], 0, 0, 0);
+  };
+  int k = 32 * wave;
+  for (; k + 32 * W * 3 < K; k += 32 * W * 4) steps(k, std::integral_constant<int, 4>());
+  for (; k < K; k += 32 * W) steps(k, std::integral_constant<int, 1>());
+#pragma unroll
+  for (int p = 0; p < PARTS; ++p) part[wave][p][lane] = make_float4(acc[p][0], acc[p][1], acc[p][2], acc[p][3]);
+  __syncthreads();
+  if (wave) return;
+  // lane (g, c): channels 16 bx + 4 g + r (r = 0..3) of token 16 by + c
+  const int t = t_b, n0 = blockIdx.x * 16 + 4 * g;
+  float y[PARTS][4];
+#pragma unroll
+  for (int p = 0; p < PARTS; ++p) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y[p][r] = n0 + r < N ? to_f32(bias[p * N + n0 + r], false) : 0.f;
+#pragma unroll
+    for (int v = 0; v < W; ++v) {
+      const float4 q = part[v][p][lane];
+      y[p][0] += q.x;
+      y[p][1] += q.y;
+      y[p][2] += q.z;
+      y[p][3] += q.w;
+    }
+  }
+  if (t >= S) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int n = n0 + r;
+    if (n >= N) break;
+    const long i = (long)t * N + n;
+    if constexpr (MODE == 0) {
+      out[i] = from_f32<false>(gelu_erf(y[0][r]));
+    } else if constexpr (MODE == 1) {
+      out[i] = from_f32<false>(__builtin_fmaf(
+          y[2][r], __builtin_fmaf(to_f32(tail.adaln[i], false), 1.0f + y[1][r], y[0][r]), to_f32(tail.pose[i], false)));
+    } else {
+      const float p = tail.first ? y[0][r] : tail.pred[i] + y[0][r];
+      tail.pred[i] = p;
+      tail.act[i] = n >= tail.n_linear && p < 0.f ? 0.f : p;
+      tail.half[i] = from_f32<false>(p);
+    }
+  }
+}
+
+static int pose_linear_check(const void* x, const void* w, const void* bias, int64_t S, int64_t N, int64_t K) {
+  QV_CHECK_ARG(S >= 0 && S <= 65535 * 16 && N > 0 && K > 0 && K % 32 == 0 && N <= INT32_MAX / 4 && K <= INT32_MAX / 4,
+               "bad shape S=%lld N=%lld K=%lld (K a multiple of 32)", (long long)S, (long long)N, (long long)K);
+  QV_CHECK_ARG(S == 0 || (x && w && bias), "null pointer argument");
+  QV_CHECK_ARG((((uintptr_t)x | (uintptr_t)w) % 16) == 0, "x and w must be 16-byte aligned");
+  return QV_OK;
+}
+
 }  // namespace qv
+
+extern "C" int qv_pose_embed(const void* src, int64_t src_stride, const void* w, const void* bias, void* out, int64_t S,
+                             int64_t N, int64_t C, void* stream) {
+  QV_CHECK_ARG(S >= 0 && S <= 65535 && N > 0 && N <= INT32_MAX - 256 && C > 0 && C <= 16 && src_stride >= 0,
+               "bad shape S=%lld N=%lld C=%lld", (long long)S, (long long)N, (long long)C);
+  if (S == 0) return QV_OK;
+  QV_CHECK_ARG(src && w && bias && out, "null pointer argument");
+  hipLaunchKernelGGL(qv::pose_embed_kernel, dim3((unsigned)((N + 255) / 256), (unsigned)S), dim3(256), 0,
+                     (hipStream_t)stream, (const uint16_t*)src, (long)src_stride, (const uint16_t*)w,
+                     (const uint16_t*)bias, (uint16_t*)out, (int)S, (int)N, (int)C);
+  return qv::check_launch("pose_embed");
+}
+
+extern "C" int qv_pose_linear_gelu(const void* x, const void* w, const void* bias, void* out, int64_t S, int64_t N,
+                                   int64_t K, void* stream) {
+  if (const int rc = qv::pose_linear_check(x, w, bias, S, N, K)) return rc;
+  if (S == 0) return QV_OK;
+  QV_CHECK_ARG(out, "null pointer argument");
+  hipLaunchKernelGGL((qv::pose_linear_kernel<0, 1>), dim3((unsigned)((N + 15) / 16), (unsigned)((S + 15) / 16)),
+                     dim3(512), 0, (hipStream_t)stream, (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias,
+                     (uint16_t*)out, (int)S, (int)N, (int)K, qv::PoseTail());
+  return qv::check_launch("pose_linear_gelu");
+}
+
+extern "C" int qv_pose_modulate(const void* e, const void* w, const void* bias, const void* adaln, const void* pose,
+                                void* x, int64_t S, int64_t D, int64_t K, void* stream) {
+  if (const int rc = qv::pose_linear_check(e, w, bias, S, D, K)) return rc;
+  if (S == 0) return QV_OK;
+  QV_CHECK_ARG(adaln && pose && x, "null pointer argument");
+  qv::PoseTail tail = {(const uint16_t*)adaln, (const uint16_t*)pose, nullptr, nullptr, nullptr, 0, 0};
+  hipLaunchKernelGGL((qv::pose_linear_kernel<1, 3>), dim3((unsigned)((D + 15) / 16), (unsigned)((S + 15) / 16)),
+                     dim3(512), 0, (hipStream_t)stream, (const uint16_t*)e, (const uint16_t*)w, (const uint16_t*)bias,
+                     (uint16_t*)x, (int)S, (int)D, (int)K, tail);
+  return qv::check_launch("pose_modulate");
+}
+
+extern "C" int qv_pose_delta(const void* x, const void* w, const void* bias, float* pred, float* act, void* half,
+                             int64_t S, int64_t cols, int64_t K, int64_t n_linear, int first, void* stream) {
+  if (const int rc = qv::pose_linear_check(x, w, bias, S, cols, K)) return rc;
+  if (S == 0) return QV_OK;
+  QV_CHECK_ARG(pred && act && half && n_linear >= 0, "null pointer argument");
+  qv::PoseTail tail = {nullptr, nullptr, pred, act, (uint16_t*)half, (int)(n_linear < cols ? n_linear : cols), first};
+  hipLaunchKernelGGL((qv::pose_linear_kernel<2, 1>), dim3((unsigned)((cols + 15) / 16), (unsigned)((S + 15) / 16)),
+                     dim3(512), 0, (hipStream_t)stream, (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias,
+                     (uint16_t*)nullptr, (int)S, (int)cols, (int)K, tail);
+  return qv::check_launch("pose_delta");
+}
 
 extern "C" int qv_pose_attention(const void* qkv, void* out, int64_t S, int64_t H, int64_t head_dim, float scale,
                                  void* stream) {

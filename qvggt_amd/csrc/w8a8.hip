@@ -641,16 +641,16 @@ extern "C" int qv_f16_gemm(const void* x, const void* w, const void* bias, const
                "x, w, gamma and out must be 16-byte and bias 8-byte aligned");
   hipStream_t st = (hipStream_t)stream;
   const int K2 = (int)K * 2;   // bytes a row
-#define QV_F16P(MT, OUT) launch<MT, OUT, false, 1, true>(x, w, nullptr, nullptr, bias, gamma, out, (int)M, (int)N, K2, st)
-#define QV_F16(MT) gamma ? QV_F16P(MT, 3) : epilogue == QV_EPI_BIAS ? QV_F16P(MT, 1) : QV_F16P(MT, 4);
+#define QV_F16_RUN(MT, OUT) launch<MT, OUT, false, 1, true>(x, w, nullptr, nullptr, bias, gamma, out, (int)M, (int)N, K2, st)
+#define QV_F16_FORM(MT) gamma ? QV_F16_RUN(MT, 3) : epilogue == QV_EPI_BIAS ? QV_F16_RUN(MT, 1) : QV_F16_RUN(MT, 4);
   switch (w8a8_form(M, N, K2, false, false)) {
-    case 41: QV_F16(4) break;
-    case 31: QV_F16(3) break;
-    case 21: QV_F16(2) break;
-    default: QV_F16(1) break;
+    case 41: QV_F16_FORM(4) break;
+    case 31: QV_F16_FORM(3) break;
+    case 21: QV_F16_FORM(2) break;
+    default: QV_F16_FORM(1) break;
   }
-#undef QV_F16
-#undef QV_F16P
+#undef QV_F16_FORM
+#undef QV_F16_RUN
   return check_launch("f16_gemm");
 }
 

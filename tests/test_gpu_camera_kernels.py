@@ -69,3 +69,50 @@ def test_pose_update(gpu, S):
 def test_empty(gpu):
     from qvggt_amd import awq_inference_engine as E
     assert E.pose_attention(torch.empty(0, 6144, device=gpu, dtype=torch.float16), 16, 0.1).shape == (0, 2048)
+
+
+@pytest.mark.parametrize("S,N,K", [(1, 1024, 2048), (8, 40, 32), (16, 1024, 2048), (17, 33, 96), (64, 1024, 288)])
+def test_pose_linears(gpu, S, N, K):
+    """The few-token fp16 linears with their tails, at token and channel
+    remainders and K below, at and above one pass of the eight waves."""
+    from qvggt_amd import awq_inference_engine as E
+    g = torch.Generator(device=gpu).manual_seed(S + N + K)
+    x = torch.randn(S, K, generator=g, device=gpu).half()
+    w = (torch.randn(3 * N, K, generator=g, device=gpu) * K ** -0.5).half()
+    b, (a, p) = torch.randn(3 * N, generator=g, device=gpu).half(), torch.randn(2, S, N, generator=g, device=gpu).half()
+    lin = x.double() @ w.double().t().contiguous() + b.double()
+    _close(E.pose_modulate(x, w, b, a, p), lin[:, 2 * N:] * (a.double() * (1 + lin[:, N:2 * N]) + lin[:, :N]) + p.double(), 20.0)
+    # gelu: the polynomial is within one fp16 step more
+    got, ref = E.pose_linear_gelu(x, w[:N], b[:N]).double(), torch.nn.functional.gelu(lin[:, :N])
+    assert ((got - ref).abs() <= ref.abs() * (2.0 ** -11 + 2.0 ** -10) + 1e-4).all()
+    pred = torch.randn(S, 9, generator=g, device=gpu)
+    want = pred.double() + lin[:, :9]
+    act, half = E.pose_delta(x, w[:9], b[:9], pred, False, 7)
+    assert ((pred.double() - want).abs() <= 1e-5 * 20).all()
+    assert torch.equal(act, torch.cat([pred[:, :7], torch.relu(pred[:, 7:])], -1)) and torch.equal(half, pred.half())
+    E.pose_delta(x, w[:9], b[:9], pred, True, 7)
+    assert ((pred.double() - lin[:, :9]).abs() <= 1e-5 * 20).all()
+
+
+def test_pose_embed(gpu):
+    from qvggt_amd import awq_inference_engine as E
+    g = torch.Generator(device=gpu).manual_seed(3)
+    w, b = torch.randn(2048, 9, generator=g, device=gpu).half(), torch.randn(2048, generator=g, device=gpu).half()
+    for src in (torch.randn(5, 9, generator=g, device=gpu).half(), torch.randn(1, 9, generator=g, device=gpu).half().expand(3, 9)):
+        e = src.double() @ w.double().t().contiguous() + b.double()
+        _close(E.pose_embed(src, w, b), torch.nn.functional.silu(e), 10.0)
+
+
+def test_camera_head_hooks_still_run(gpu):
+    """A hook on one of the head's own linears sends the forward through the
+    module calls (so the hook sees its output), with the fused path's result."""
+    from qvggt_amd.camera_head import CameraHead
+    head = CameraHead.random(seed=2, device=gpu)
+    t = torch.randn(3, 2048, generator=torch.Generator(device=gpu).manual_seed(1), device=gpu).half()
+    plain, seen = head(t), []
+    handle = head.pose_branch.fc1.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+    hooked = head(t)
+    handle.remove()
+    assert seen == [(3, 1024)] * 4
+    for a, b in zip(plain, hooked):
+        assert (a - b).abs().max().item() <= 1e-2 * b.abs().max().item()
