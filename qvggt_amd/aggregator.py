@@ -273,6 +273,11 @@ def _affine(ln: nn.Module):
         return ln.weight, ln.bias
 
 
+def _aligned(*tensors: torch.Tensor) -> bool:
+    """Whether the fp16 linear's 16-byte accesses may read and write them."""
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def _with_depth(cfg: AggregatorConfig, depth: int | None) -> AggregatorConfig:
     return cfg if depth is None else dataclasses.replace(cfg, depth=depth, dino_depth=depth)
 
@@ -383,9 +388,18 @@ class DinoBlock(nn.Module):
         qkv = torch.addmm(qkv_b, h, qkv_w.t(), out=ws["qkv"])
         v3 = qkv.view(M, 3, HEADS, HEAD_DIM)
         att = E.attention(*v3.unbind(1), TOKENS, out=ws["att"].view(M, HEADS, HEAD_DIM))
-        E.f16_linear(att.view(M, DIM), *_affine(attn.proj), out=x, gamma=self.ls1.gamma)
+        proj_w, proj_b = _affine(attn.proj)
+        gamma1 = self.ls1.gamma
+        if x.is_contiguous() and _aligned(x, att, proj_w, proj_b, gamma1):
+            E.f16_linear(att.view(M, DIM), proj_w, proj_b, out=x, gamma=gamma1)
+        else:
+            x.addcmul_(torch.addmm(proj_b, att.view(M, DIM), proj_w.t(), out=ws["o"]), gamma1)
         h = E.layer_norm(x, *_affine(self.norm2), self.eps, out=ws["h"])
-        f = E.f16_linear(h, *_affine(mlp.fc1), QV_EPI_BIAS_GELU, out=ws["f"])
+        fc1_w, fc1_b = _affine(mlp.fc1)
+        if _aligned(h, fc1_w, fc1_b, ws["f"]):
+            f = E.f16_linear(h, fc1_w, fc1_b, QV_EPI_BIAS_GELU, out=ws["f"])
+        else:
+            f = F.gelu(torch.addmm(fc1_b, h, fc1_w.t(), out=ws["f"]))
         o = torch.addmm(fc2_b, f, fc2_w.t(), out=ws["o"])
         x.addcmul_(o, self.ls2.gamma)
         return x

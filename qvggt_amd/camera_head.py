@@ -61,7 +61,8 @@ POSE_LINEAR_MAX = 64
 
 def _plain(*modules) -> bool:
     """Whether calling the modules does nothing but their own forward: no hooks
-    on them or on all modules, the linears plain fp16 ones with a bias."""
+    on them or on all modules, the linears plain fp16 ones with a bias and
+    weights that 16-byte loads can read."""
     g = nn.modules.module
     if g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks:
         return False
@@ -71,7 +72,8 @@ def _plain(*modules) -> bool:
         if isinstance(m, nn.Linear):
             p = m._parameters
             if (type(m) is not nn.Linear or p.get("weight") is None or p.get("bias") is None
-                    or p["weight"].dtype != torch.float16 or p["bias"].dtype != torch.float16):
+                    or p["weight"].dtype != torch.float16 or p["bias"].dtype != torch.float16
+                    or p["weight"].data_ptr() % 16):
                 return False
         elif type(m) not in (nn.Sequential, nn.SiLU):
             return False

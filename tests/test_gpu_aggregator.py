@@ -204,3 +204,25 @@ def test_checkpoint_config_eps_reaches_the_kernels(gpu, tmp_path):
         ref = OA.aa_block_delta(x0, _params(blk), AG.TOKENS, pos.cpu().numpy(), c, s, rows, eps=eps)
         errs[eps] = np.abs(got - ref).max() / np.abs(ref).max()
     assert errs[1e-5] <= 1e-2 and errs[1e-6] > 5e-2, errs
+
+
+def test_dino_block_takes_strided_and_unaligned_tensors(gpu):
+    """A residual stream with row gaps and weights off 16-byte addresses keep
+    the library's linears, within two fp16 steps of the fused path's result."""
+    from qvggt_amd import aggregator as AG
+    agg = AG.Aggregator.random(seed=6, device=gpu, depth=1)
+    blk, M = agg.patch_embed.blocks[0], AG.TOKENS
+    ws = agg._workspace(M, gpu)
+    blk.ls1.gamma.fill_(0.5)
+    blk.ls2.gamma.fill_(0.5)
+    x = torch.randn(M, AG.DIM, generator=torch.Generator(device=gpu).manual_seed(2), device=gpu).half()
+    want = blk(x.clone(), ws)
+    wide = torch.zeros(M, AG.DIM + 8, device=gpu, dtype=torch.float16)
+    wide[:, :AG.DIM] = x
+    got = blk(wide[:, :AG.DIM], ws)
+    for l in (blk.attn.proj, blk.mlp.fc1):
+        w = torch.empty(l.weight.numel() + 1, device=gpu, dtype=torch.float16)[1:].view_as(l.weight)
+        l.weight = torch.nn.Parameter(w.copy_(l.weight), requires_grad=False)
+    off = blk(x.clone(), ws)
+    for y in (got, off):
+        assert (y.float() - want.float()).abs().max().item() <= 2.0 ** -9 * want.float().abs().max().item()
