@@ -333,6 +333,18 @@ int qv_attention_fwd(const void* q, const void* k, const void* v, void* out, int
 int qv_f16_gemm(const void* x, const void* w, const void* bias, const void* gamma, void* out,
                 int64_t M, int64_t N, int64_t K, int epilogue, void* stream);
 
+/*
+ * W4A16 linear of LayerNorm(x) for few tokens (a camera-head trunk block's
+ * norm + qkv, norm + fc1): fp16, M <= 16, K <= 2048 a multiple of 128, N a
+ * multiple of 32; ln_weight / ln_bias (K); epilogue QV_EPI_BIAS or
+ * QV_EPI_BIAS_GELU.  What qv_layernorm then qv_w4a16_gemm compute, the norm's
+ * statistics summed in another order.
+ */
+int qv_w4a16_ln_linear(const void* x, const void* ln_weight, const void* ln_bias, float eps,
+                       const void* qweight, const void* scales, const void* scaled_zeros,
+                       const void* bias, void* out, int64_t M, int64_t N, int64_t K, int epilogue,
+                       void* stream);
+
 /* ---------------------------------------------------- camera head
  * No counterparts in the reference extension: the camera head's graph is in
  * the external vggt-hf (qvggt/inference/loader.py:204-206 quantises its trunk

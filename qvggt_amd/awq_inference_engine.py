@@ -68,9 +68,10 @@ def _on_gpu(*tensors: torch.Tensor, what: str) -> int:
     return dev
 
 
-# The call path of an op is Python, so its cost (17 us for a linear when each
-# pointer and the stream were wrapped in objects, 8-9 us now) bounds small launches: the
-# pointers, the stream and the device go to ctypes as plain integers.
+# The call path of an op is Python, so its cost (18 us for a ``WQLinear``
+# call when each pointer and the stream were wrapped in objects, 12.8 us now)
+# bounds small launches: the pointers, the stream and the device go to ctypes as
+# plain integers.
 def _ptr(t: torch.Tensor | None):
     return t.data_ptr() if t is not None else None
 
@@ -241,6 +242,30 @@ def w4a16_linear_residual(x: torch.Tensor, qweight: torch.Tensor, scales: torch.
         _lib.call("qv_w4a16_gemm_residual", _ptr(x), _ptr(qw), _ptr(sc), _ptr(sz), _ptr(bb), _ptr(gg),
                   _ptr(residual), M, N, K, dt, _stream(dev))
     return residual
+
+
+def w4a16_ln_linear(x: torch.Tensor, ln_weight: torch.Tensor, ln_bias: torch.Tensor, eps: float,
+                    qweight: torch.Tensor, scales: torch.Tensor, scaled_zeros: torch.Tensor, bias: torch.Tensor,
+                    epilogue: int) -> torch.Tensor:
+    """``w4a16_linear(layer_norm(x, ...), ..., bias, epilogue)`` in one kernel for
+    x (M <= 16, K <= 2048) fp16; epilogue bias or bias + GELU."""
+    what = "w4a16_ln_linear"
+    if x.dtype != torch.float16 or x.dim() != 2:
+        _fail(f"{what}: x must be float16 (M, K)")
+    M, K = x.shape
+    N = qweight.shape[0] * 4
+    _check_w4_tables(qweight, scales, scaled_zeros, N, K, x.dtype, what)
+    for name, t, n in (("bias", bias, N), ("ln_weight", ln_weight, K), ("ln_bias", ln_bias, K)):
+        if t.dtype != x.dtype or t.numel() != n:
+            _fail(f"{what}: {name} must be ({n},) {x.dtype}")
+    dev = _on_gpu(x, ln_weight, ln_bias, qweight, scales, scaled_zeros, bias, what=what)
+    x, lw, lb = _contig(x), _contig(ln_weight), _contig(ln_bias)
+    out = x.new_empty((M, N))
+    qw, sc, sz, bb = _contig(qweight), _contig(scales), _contig(scaled_zeros), _contig(bias)
+    with _device(dev):
+        _lib.call("qv_w4a16_ln_linear", _ptr(x), _ptr(lw), _ptr(lb), eps, _ptr(qw), _ptr(sc), _ptr(sz), _ptr(bb),
+                  _ptr(out), M, N, K, epilogue, _stream(dev))
+    return out
 
 
 def w4a16_plan(M: int, N: int, K: int, epilogue: int = _lib.QV_EPI_NONE) -> dict:

@@ -38,7 +38,8 @@ import torch.nn.functional as F
 
 from . import awq_inference_engine as E
 from ._lib import QV_EPI_BIAS, QV_EPI_BIAS_GELU
-from .aggregator import LayerScale, Mlp, _affine, _linear, _linear_residual, quantize_w4
+from .aggregator import LayerScale, Mlp, _affine, _aligned, _linear, _linear_residual, quantize_w4
+from .awq.qmodule import WQLinear, w4_buffers
 
 DIM = 2048
 HEADS = 16
@@ -80,6 +81,19 @@ def _plain(*modules) -> bool:
     return True
 
 
+def _norm_linear(norm, layer, x: torch.Tensor, epilogue: int, n: int) -> torch.Tensor:
+    """layer(norm(x)) with its bias (+ GELU): one kernel for a ``WQLinear`` on up
+    to 16 tokens (one MFMA tile; 6.3-9.0 us against 7.5-9.5 for the two, and
+    one call less), else the norm, then the linear."""
+    if 0 < x.shape[0] <= 16 and isinstance(layer, WQLinear) and x.dtype == torch.float16:
+        qweight, scales, scaled_zeros, bias = w4_buffers(layer)
+        weight, shift = _affine(norm)
+        if bias is not None and qweight.shape[0] * 4 == n and _aligned(x, weight, shift):
+            return E.w4a16_ln_linear(x, weight, shift, LN_EPS, qweight, scales, scaled_zeros, bias, epilogue)
+    h = E.layer_norm(x, *_affine(norm), LN_EPS)
+    return _linear(layer, h, epilogue, x.new_empty((x.shape[0], n)))
+
+
 class TrunkBlock(nn.Module):
     """Camera-head trunk block: LN -> qkv -> attention over the frames -> proj ->
     LayerScale residual; LN -> fc1 -> GELU -> fc2 -> LayerScale residual."""
@@ -99,8 +113,7 @@ class TrunkBlock(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         S = x.shape[0]
         attn, mlp = self.attn, self.mlp
-        h = E.layer_norm(x, *_affine(self.norm1), LN_EPS)
-        qkv = _linear(attn.qkv, h, QV_EPI_BIAS, x.new_empty((S, 3 * DIM)))
+        qkv = _norm_linear(self.norm1, attn.qkv, x, QV_EPI_BIAS, 3 * DIM)
         if S <= POSE_ATTENTION_MAX:
             att = E.pose_attention(qkv, HEADS, HEAD_DIM ** -0.5)
         else:
@@ -109,8 +122,7 @@ class TrunkBlock(nn.Module):
             att = a.permute(1, 0, 2).reshape(S, DIM).half()
         o = x.new_empty((S, DIM))   # for a linear that is not fused with its residual update
         _linear_residual(attn.proj, att, self.ls1.gamma, x, o)
-        h = E.layer_norm(x, *_affine(self.norm2), LN_EPS)
-        f = _linear(mlp.fc1, h, QV_EPI_BIAS_GELU, x.new_empty((S, MLP_DIM)))
+        f = _norm_linear(self.norm2, mlp.fc1, x, QV_EPI_BIAS_GELU, MLP_DIM)
         _linear_residual(mlp.fc2, f, self.ls2.gamma, x, o)
         return x
 

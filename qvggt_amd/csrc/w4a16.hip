@@ -228,6 +228,118 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(MB * NB ==
   }
 }
 
+// The unsplit skinny product (fp16, 16 tokens, 32 channels a workgroup, one
+// 128-k group a wave: K <= 2048) of LayerNorm(x): every workgroup normalises
+// the at most 64 KB of x itself, a wave per token row for the statistics
+// (fp32, two-pass), each wave then its own fragments, rounded to fp16 as
+// layernorm_kernel's output is.  The weights are requested before the
+// statistics, which run under their latency.  For a trunk block's norm + qkv
+// and norm + fc1, which as two launches are bound by the launches.  Weights cold,
+// us, against LayerNorm then the skinny kernel: 2048 -> 6144 at M = 1 6.3 (7.5),
+// 4 6.5 (8.1), 8 7.0 (8.5), 16 8.6 (9.3); 2048 -> 8192 + GELU at M = 1 6.7
+// (7.9), 8 7.3 (8.9), 16 9.0 (9.5); and one call of ~10 us on the host less.
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void w4a16_ln_skinny_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ ln_w, const uint16_t* __restrict__ ln_b, float eps,
+    const uint32_t* __restrict__ qw, const uint16_t* __restrict__ scales, const uint16_t* __restrict__ zeros,
+    const uint16_t* __restrict__ bias, uint16_t* __restrict__ out, int M, int N, int K, int gelu) {
+  constexpr int NB = 2;
+  __shared__ f32x4 red[16][64];
+  __shared__ float2 stat[16];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nwaves = blockDim.x >> 6;
+  const int g = lane >> 4, li = lane & 15;
+  const int n0 = blockIdx.x * 16 * NB;
+  const uint32_t K2 = (uint32_t)K * 2;
+  const auto rsX = make_rsrc(x, (uint64_t)M * K2);
+  uint4 wq[NB], xb[4];
+  uint32_t sj[NB], zj[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int n = n0 + 16 * j + li;
+    wq[j] = *reinterpret_cast<const uint4*>(qw + qw_chunk_u32(n, wave, g, K));
+    sj[j] = scales[(size_t)wave * N + n];
+    zj[j] = zeros[(size_t)wave * N + n];
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t) xb[t] = buf_load16(rsX, (uint32_t)li * K2 + (uint32_t)g * 64, wave * 256 + t * 16);
+  // ---- row statistics: lane l holds halves 512 c + 8 l .. + 7 of the row
+  for (int r = wave; r < M; r += nwaves) {
+    uint4 u[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {   // past the row: zeros (not counted below)
+      const int e = 512 * c + 8 * lane;
+      u[c] = e < K ? *reinterpret_cast<const uint4*>(x + (size_t)r * K + e) : make_uint4(0, 0, 0, 0);
+    }
+    float sum = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const uint32_t w[4] = {u[c].x, u[c].y, u[c].z, u[c].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sum = mix_add<0>(w[e], sum);
+        sum = mix_add<1>(w[e], sum);
+      }
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) sum += __shfl_xor(sum, d);
+    const float nm = -(sum / (float)K);
+    float sq = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const uint32_t w[4] = {u[c].x, u[c].y, u[c].z, u[c].w};
+      if (512 * c + 8 * lane < K) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float d0 = mix_add<0>(w[e], nm), d1 = mix_add<1>(w[e], nm);
+          sq = __builtin_fmaf(d0, d0, sq);
+          sq = __builtin_fmaf(d1, d1, sq);
+        }
+      }
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) sq += __shfl_xor(sq, d);
+    if (lane == 0) stat[r] = make_float2(nm, 1.0f / __builtin_sqrtf(sq / (float)K + eps));
+  }
+  __syncthreads();
+  // ---- this wave's fragments, normalised (tokens past M: not stored)
+  const float2 ms = stat[li < M ? li : 0];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int k = 128 * wave + 32 * g + 8 * t;
+    const uint4 gv = *reinterpret_cast<const uint4*>(ln_w + k), bv = *reinterpret_cast<const uint4*>(ln_b + k);
+    const uint32_t xw[4] = {xb[t].x, xb[t].y, xb[t].z, xb[t].w}, gw[4] = {gv.x, gv.y, gv.z, gv.w},
+                   bw[4] = {bv.x, bv.y, bv.z, bv.w};
+    uint32_t y[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      y[e] = pack2<false>(mix_add<0>(bw[e], mix_mul<0>(mix_add<0>(xw[e], ms.x) * ms.y, gw[e])),
+                          mix_add<1>(bw[e], mix_mul<1>(mix_add<1>(xw[e], ms.x) * ms.y, gw[e])));
+    xb[t] = make_uint4(y[0], y[1], y[2], y[3]);
+  }
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    f32x4 acc = (f32x4){0.f, 0.f, 0.f, 0.f};
+    acc = mfma16<false>(dq_frag<false, 0>(wq[j], sj[j], zj[j]), xb[0], acc);
+    acc = mfma16<false>(dq_frag<false, 1>(wq[j], sj[j], zj[j]), xb[1], acc);
+    acc = mfma16<false>(dq_frag<false, 2>(wq[j], sj[j], zj[j]), xb[2], acc);
+    acc = mfma16<false>(dq_frag<false, 3>(wq[j], sj[j], zj[j]), xb[3], acc);
+    if (j) __syncthreads();
+    red[wave][lane] = acc;
+    __syncthreads();
+    for (int e = tid; e < 256; e += blockDim.x) {
+      const int l = (e >> 2) & 63, r = e & 3, m = l & 15, n = n0 + 16 * j + 4 * (l >> 4) + r;
+      if (m >= M) continue;
+      float v = 0.f;
+      for (int w = 0; w < nwaves; ++w) v += red[w][l][r];
+      v += to_f32(bias[n], false);
+      if (gelu) v = gelu_erf(v);
+      out[(size_t)m * N + n] = from_f32<false>(v);
+    }
+  }
+}
+
 // ---------------------------------------------------------- dequant kernel
 // One thread per (row n, 32-k chunk): writes 32 weights in natural k order.
 template <bool BF16>
@@ -913,6 +1025,27 @@ extern "C" int qv_w4a16_gemm_residual(const void* x, const void* qweight, const 
                              QV_EPI_BIAS_RESID, st, gamma);
   return launch_gemm<false>(x, qweight, scales, scaled_zeros, bias, residual, (int)M, (int)N, (int)K,
                             QV_EPI_BIAS_RESID, st, gamma);
+}
+
+extern "C" int qv_w4a16_ln_linear(const void* x, const void* ln_weight, const void* ln_bias, float eps,
+                                  const void* qweight, const void* scales, const void* scaled_zeros, const void* bias,
+                                  void* out, int64_t M, int64_t N, int64_t K, int epilogue, void* stream) {
+  QV_CHECK_ARG(M >= 0 && M <= 16 && N > 0 && N % 32 == 0 && N <= INT32_MAX && K >= 128 && K % 128 == 0 && K <= 2048,
+               "bad shape M=%lld N=%lld K=%lld (M <= 16, N a multiple of 32, K of 128 and at most 2048)", (long long)M,
+               (long long)N, (long long)K);
+  QV_CHECK_ARG(epilogue == QV_EPI_BIAS || epilogue == QV_EPI_BIAS_GELU, "unsupported epilogue %d", epilogue);
+  if (M == 0) return QV_OK;
+  QV_CHECK_ARG(x && ln_weight && ln_bias && qweight && scales && scaled_zeros && bias && out, "null pointer argument");
+  QV_CHECK_ARG((((uintptr_t)x | (uintptr_t)ln_weight | (uintptr_t)ln_bias | (uintptr_t)qweight) % 16) == 0,
+               "x, the norm's weights and qweight must be 16-byte aligned");
+  QV_CHECK_ARG((((uintptr_t)scales | (uintptr_t)scaled_zeros) % 4) == 0 && ((uintptr_t)bias % 8) == 0,
+               "scale tables must be 4-byte and bias 8-byte aligned");
+  hipLaunchKernelGGL(qv::w4a16_ln_skinny_kernel, dim3((unsigned)(N / 32)), dim3((unsigned)(K / 128 * 64)), 0,
+                     (hipStream_t)stream, (const uint16_t*)x, (const uint16_t*)ln_weight, (const uint16_t*)ln_bias, eps,
+                     (const uint32_t*)qweight, (const uint16_t*)scales, (const uint16_t*)scaled_zeros,
+                     (const uint16_t*)bias, (uint16_t*)out, (int)M, (int)N, (int)K,
+                     epilogue == QV_EPI_BIAS_GELU ? 1 : 0);
+  return qv::check_launch("w4a16_ln_linear");
 }
 
 extern "C" int qv_w4a16_gemm_qkrope(const void* x, const void* qweight, const void* scales,

@@ -116,3 +116,28 @@ def test_camera_head_hooks_still_run(gpu):
     assert seen == [(3, 1024)] * 4
     for a, b in zip(plain, hooked):
         assert (a - b).abs().max().item() <= 1e-2 * b.abs().max().item()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 32, 128), (5, 6144, 2048), (8, 8192, 2048), (16, 64, 1920), (13, 4096, 640), (7, 96, 384)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_w4a16_ln_linear(gpu, M, N, K, gelu):
+    """LayerNorm + W4A16 linear in one kernel against the two ops: the norm's
+    fp16 output differs by at most one step in a few places (its fp32 sums run
+    in another order, moving a value by 1e-6 of its size), so the sums differ by
+    that share of a step, 2^-11 * sqrt(K) of the typical term, and the output by
+    one more rounding."""
+    from qvggt_amd import awq_inference_engine as E
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    x = (torch.randn(M, K, generator=g, device=gpu) * 3 + 1).half()
+    w, b = (1 + 0.1 * torch.randn(K, generator=g, device=gpu)).half(), (0.1 * torch.randn(K, generator=g, device=gpu)).half()
+    qw = torch.randint(-32768, 32768, (N // 4, K), generator=g, device=gpu, dtype=torch.int32).to(torch.int16)
+    rows = (K // 128 + 7) // 8 * 8
+    s = (torch.rand(rows, N, generator=g, device=gpu) * 0.01 + 0.005).half()
+    z = -(s.float() * 7).half()
+    bias = torch.randn(N, generator=g, device=gpu).half()
+    got = E.w4a16_ln_linear(x, w, b, 1e-5, qw, s, z, bias, 2 if gelu else 1).double()
+    h = E.layer_norm(x, w, b, 1e-5)
+    lin = h.double() @ E.w4a16_dequantize(qw, s, z, K).double().t().contiguous() + bias.double()
+    ref = torch.nn.functional.gelu(lin) if gelu else lin
+    term = (h.double().abs().mean() * 0.05)
+    assert ((got - ref).abs() <= ref.abs() * 2.0 ** -10 + term * 2.0 ** -11 * K ** 0.5 + 1e-4).all()
