@@ -15,11 +15,13 @@
 // The softmax is trimmed to what the MFMAs cannot hide: key masking only on
 // the last (partial) tile; Q pre-scaled by scale * log2(e) and the score
 // accumulators started at -m (the running reference), so P = 2^S takes one
-// exp2 per score and nothing else; row sums by one fp32 add per score (a
-// v_dot2 of the packed fp16 pair is one instruction instead of two, but beside
-// MFMAs in flight it cost ~16 cycles: a 32 x 64 tile's 16 MFMAs, 32 exp2 and
-// packs took 527 cycles alone, 781 with 16 v_dot2, 541 with 32 adds; 43968
-// tokens 7.87 -> 7.74 ms, 10992 541 -> 526 us, same box);
+// exp2 per score and nothing else; row sums by v_dot2 on
+// the fp16 pairs that the PV product uses, so that P's rounding cancels in the
+// quotient (fp32 adds of the unrounded P raised the error against 64 bits by
+// 2-4 % at sharp scores: 300 tokens, q scaled 4 times, 4.82e-4 -> 5.01e-4; same
+// box, they took 7.17 ms against 7.13 at 43968 tokens, 94.3 us against 96.2 at
+// 4122, 47.8 against 49.1 at 2748; v_fma_mix_f32 adds of the fp16 values were
+// 1-3 % slower than the unrounded ones from 4122 tokens on);
 // and a lazy rescale -- the reference moves only when a tile exceeds it by
 // 2^8, so most tiles skip the O *= alpha pass, and the tile maximum itself is
 // only computed when a lane's tile sum says some P may have exceeded 2^8.
@@ -252,16 +254,17 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(QB =
       const float p0 = __builtin_amdgcn_exp2f(shift ? s0 + off : s0);
       const float p1 = __builtin_amdgcn_exp2f(shift ? s1 + off : s1);
       const f16x2 ph = {(_Float16)p0, (_Float16)p1};
-      t += p0;
-      t += p1;
       return __builtin_bit_cast(uint32_t, ph);
+    };
+    auto add_p = [&](uint32_t w) __attribute__((always_inline)) {
+      t = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, w), (f16x2){(_Float16)1.0f, (_Float16)1.0f}, t, false);
     };
     auto set_p = [&](int qb, const uint32_t (&pw)[16]) __attribute__((always_inline)) {
 #pragma unroll
       for (int st = 0; st < 4; ++st) pf[qb][st] = make_uint4(pw[4 * st], pw[4 * st + 1], pw[4 * st + 2], pw[4 * st + 3]);
     };
     // P = 2^S' = 2^(S - m_use) of a query block in fp16 against the current
-    // reference, with the tile's partial row sum t (of the fp32 values).  The
+    // reference, with the tile's partial row sum t (of the fp16 values).  The
     // tile maximum is only needed when some P could exceed 2^RESCALE_SLACK,
     // and every such P makes t exceed it too (P >= 0), so the maximum is
     // computed only for waves where some lane's t does, and on the first tile
@@ -270,7 +273,9 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(QB =
     // that block 1's QK MFMAs run beside block 0's exp2 and block 0's PV MFMAs
     // beside block 1's (left to the compiler the MFMAs clustered: 10992 tokens
     // 488 -> 481 us, 8 x 1374 75.2 -> 73.0, 43968 7.12 -> 7.07 ms, the same
-    // bits; at QB = 1 fencing cost 5 % at 1 x 1374 and is left out).
+    // bits; at QB = 1 fencing cost 5 % at 1 x 1374 and is left out).  A
+    // group's sums come one group later, at QB = 1 after all groups (in the
+    // group itself 1 x 4122 took 2 % more, 1 x 2748 3 %).
     auto softmax = [&](int qb, auto&& slot) __attribute__((always_inline)) {
       if (mask) mask_keys(qb);
       uint32_t pw[16];
@@ -279,10 +284,16 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(QB =
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         slot(i);
+        if (QB == 2 && i > 0) {
+          add_p(pw[2 * i - 2]);
+          add_p(pw[2 * i - 1]);
+        }
         pw[2 * i] = p_word(qb, 2 * i, false, 0.f);
         pw[2 * i + 1] = p_word(qb, 2 * i + 1, false, 0.f);
         if constexpr (QB == 2) __builtin_amdgcn_sched_barrier(0);
       }
+#pragma unroll
+      for (int w = QB == 2 ? 14 : 0; w < 16; ++w) add_p(pw[w]);
       if (__builtin_amdgcn_ballot_w64(!(t <= P_SUM_LIMIT) || m_use[qb] == -INFINITY)) {
         // ---- tile maximum of this query (both lane halves hold 32 keys each)
         float mx = sc[qb][0][0];
@@ -305,6 +316,8 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(QB =
           const float off = base[qb] - m_new;
 #pragma unroll
           for (int w = 0; w < 16; ++w) pw[w] = p_word(qb, w, true, off);
+#pragma unroll
+          for (int w = 0; w < 16; ++w) add_p(pw[w]);
         }
         base[qb] = m_use[qb];
       }

@@ -98,6 +98,26 @@ def test_attention_fine_and_wide_forms_agree_bitwise(gpu, L):
     assert np.abs(two.float().cpu().numpy() - ref).max() / np.abs(ref).max() <= TOL
 
 
+@pytest.mark.parametrize("B,L", [(1, 64), (3, 300), (64, 300), (1, 1374), (24, 1374)])
+@pytest.mark.parametrize("sharp", [1.0, 4.0, 8.0])
+def test_attention_weights_sum_to_one(gpu, B, L, sharp):
+    """With one value vector for all keys the output is that vector, however
+    the probabilities round: the row sums take the fp16 probabilities that the
+    PV product uses.  Both are fp32 sums of at most 1374 positive terms, so
+    their quotient is off by under 1374 * 2^-23 < 2^-12, which rounds back to
+    the fp16 value exactly.  (Sums of the unrounded probabilities leave up to
+    2^-11 where one key dominates.)  Both forms, q scaled up to 8 times."""
+    from qvggt_amd import awq_inference_engine as E
+    H = 16
+    g = torch.Generator(device=gpu).manual_seed(B + L)
+    x = torch.randn(B * L, 3, H, 64, generator=g, device=gpu)
+    x[:, 0] *= sharp
+    x[:, 2] = torch.randn(1, H, 64, generator=g, device=gpu)
+    x = x.half()
+    out = E.attention(x[:, 0], x[:, 1], x[:, 2], L)
+    assert torch.equal(out, x[:, 2])
+
+
 def test_attention_separate_buffers_and_determinism(gpu):
     from qvggt_amd import awq_inference_engine as E
     B, L, H = 2, 300, 4
