@@ -263,7 +263,7 @@ __global__ __launch_bounds__(512) void pose_linear_kernel(const uint16_t* __rest
     if (n >= N) break;
     const long i = (long)t * N + n;
     if constexpr (MODE == 0) {
-      out[i] = from_f32<false>(gelu_erf(y[0][r]));
+      out[i] = from_f32<false>(gelu_erf_fine(y[0][r]));
     } else if constexpr (MODE == 1) {
       out[i] = from_f32<false>(__builtin_fmaf(
           y[2][r], __builtin_fmaf(to_f32(tail.adaln[i], false), 1.0f + y[1][r], y[0][r]), to_f32(tail.pose[i], false)));

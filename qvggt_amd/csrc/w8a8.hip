@@ -422,7 +422,7 @@ void w8a8_gemm_kernel(const int8_t* __restrict__ a, const int8_t* __restrict__ b
             float t = (float)acc[j][i][4 * qd + e];
             if constexpr (!F16) t = t * wsn[e] * am[i];
             if constexpr (BIAS) t = t + bn[e];
-            if constexpr (OUT == 4) t = gelu_erf(t);
+            if constexpr (OUT == 4) t = gelu_erf_fine(t);
             // keep the fp32 rounding of t: without this the backend fuses the last
             // multiply and the fp16 conversion into one v_fma_mixlo_f16 (one rounding)
             asm volatile("" : "+v"(t));
@@ -621,8 +621,8 @@ static int w8a8_run(const void* a, const void* b, const void* ws, const void* as
 // estimate, K in bytes a row).  Bound by LDS bandwidth: both operands pass
 // through it, 6 KB of fragments per 8 MFMAs a wave plus the copies, ~140 bytes
 // a clock at full MFMA rate against 128.  What it gains over the library's
-// product is the fused epilogue: bias + GELU 1024 -> 4096 in 64.5 us against
-// 63 + 17 at M = 5496 (22 / 29 at 1374, 100 / 112 at 8244, 220 / 260 at 21984),
+// product is the fused epilogue: bias + GELU 1024 -> 4096 in 65.6 us against
+// 81 at M = 5496 (22.9 / 28.4 at 1374, 99.9 / 114 at 8244, 222 / 262 at 21984),
 // bias + residual 1024 -> 1024 in 25.2 against 18.5 + 9.5.  Without one (qkv),
 // or at K = 4096, the library's product is faster (43 / 52 us, 49 / 77).
 extern "C" int qv_f16_gemm(const void* x, const void* w, const void* bias, const void* gamma, void* out, int64_t M,

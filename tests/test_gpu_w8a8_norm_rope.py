@@ -607,3 +607,26 @@ def test_f16_linear(gpu, M, N, K, mode):
     strided[:, :K] = x
     if mode == "bias":
         assert torch.equal(E.f16_linear(strided[:, :K], w, b), got)
+
+
+def test_f16_gelu_every_fp16_input(gpu):
+    """The GELU of the fp16 linears (``f16_linear`` and the camera head's
+    ``pose_linear_gelu``) at every finite fp16 value of the linear, against
+    float64: one fp16 rounding (2^-11 relative, 2^-25 below the normal range)
+    plus the 3e-6 that the fitted tail may be off, a few fp32 roundings (2^-20)
+    and nothing more; inf, -inf and NaN as torch's GELU gives them."""
+    from qvggt_amd import awq_inference_engine as E
+    v = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.float16).to(gpu)
+    v = torch.cat([v[torch.isfinite(v)], torch.tensor([float("inf"), float("-inf"), float("nan")], device=gpu).half()])
+    x = torch.zeros(v.numel(), 32, device=gpu, dtype=torch.float16)
+    x[:, 0] = v
+    w = torch.zeros(16, 32, device=gpu, dtype=torch.float16)
+    w[:, 0] = 1
+    b = torch.zeros(16, device=gpu, dtype=torch.float16)
+    vd = v[:-3].double()
+    ref = 0.5 * vd * torch.special.erfc(-vd * 0.5 ** 0.5)
+    for got in (E.f16_linear(x, w, b, 2), E.pose_linear_gelu(x, w, b)):
+        err = (got[:-3, 0].double() - ref).abs()
+        assert (err <= ref.abs() * (2.0 ** -11 + 3e-6 + 2.0 ** -20) + 2.0 ** -25).all()
+        assert torch.equal(got[:-2], got[:-2, :1].expand(-1, 16))
+        assert got[-3, 0].item() == float("inf") and got[-2:].isnan().all()
