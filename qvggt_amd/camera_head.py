@@ -47,6 +47,7 @@ HEAD_DIM = DIM // HEADS      # 128
 MLP_DIM = 4 * DIM
 TRUNK_DEPTH = 4
 POSE_DIM = 9                 # absT (3) + quaternion (4) + FoV (2)
+POSE_LINEAR = 7              # leading columns without an activation (translation, quaternion)
 LN_EPS = 1e-5               # token_norm, trunk_norm, trunk blocks (torch's default)
 ADALN_EPS = 1e-6
 # Frames up to which the pose attention runs in its one fp32 kernel; above, the
@@ -92,6 +93,11 @@ def _norm_linear(norm, layer, x: torch.Tensor, epilogue: int, n: int) -> torch.T
             return E.w4a16_ln_linear(x, weight, shift, LN_EPS, qweight, scales, scaled_zeros, bias, epilogue)
     h = E.layer_norm(x, *_affine(norm), LN_EPS)
     return _linear(layer, h, epilogue, x.new_empty((x.shape[0], n)))
+
+
+def activate_pose(enc: torch.Tensor) -> torch.Tensor:
+    """absT_quaR_FoV with linear translation / quaternion and ReLU field of view."""
+    return torch.cat([enc[..., :POSE_LINEAR], F.relu(enc[..., POSE_LINEAR:])], dim=-1)
 
 
 class TrunkBlock(nn.Module):
@@ -192,10 +198,9 @@ class CameraHead(nn.Module):
         [frame | global] aggregator output: the head's input."""
         return layer_out[:, 0].contiguous()
 
-    @staticmethod
-    def activate(enc: torch.Tensor) -> torch.Tensor:
-        """absT_quaR_FoV with linear translation / quaternion and ReLU field of view."""
-        return torch.cat([enc[..., :7], F.relu(enc[..., 7:])], dim=-1)
+    # the pose update's kernels hold this one; another (a subclass's, an
+    # instance's) is called on the prediction
+    activate = staticmethod(activate_pose)
 
     @torch.no_grad()
     def forward(self, tokens: torch.Tensor, num_iterations: int = 4):
@@ -207,7 +212,9 @@ class CameraHead(nn.Module):
         pred = torch.empty(S, POSE_DIM, dtype=torch.float32, device=tokens.device)
         outs = []
         embed, modulation, fc1, fc2 = self.embed_pose, self.poseLN_modulation, self.pose_branch.fc1, self.pose_branch.fc2
-        fused = S <= POSE_LINEAR_MAX and _plain(embed, modulation, *modulation, fc1, fc2) and not torch.is_autocast_enabled()
+        kernel_act = self.activate is activate_pose
+        fused = (kernel_act and S <= POSE_LINEAR_MAX and _plain(embed, modulation, *modulation, fc1, fc2)
+                 and not torch.is_autocast_enabled())
         for i in range(num_iterations):
             if fused:
                 x = E.pose_modulate(E.pose_embed(src, *_affine(embed)), *_affine(modulation[1]), adaln, pose)
@@ -217,9 +224,13 @@ class CameraHead(nn.Module):
                 blk(x)
             h = E.layer_norm(x, *_affine(self.trunk_norm), LN_EPS)
             if fused:
-                act, src = E.pose_delta(E.pose_linear_gelu(h, *_affine(fc1)), *_affine(fc2), pred, i == 0, 7)
+                act, src = E.pose_delta(E.pose_linear_gelu(h, *_affine(fc1)), *_affine(fc2), pred, i == 0, POSE_LINEAR)
+            elif kernel_act:
+                act, src = E.pose_update(fc2(F.gelu(fc1(h))), pred, i == 0, POSE_LINEAR)
             else:
-                act, src = E.pose_update(fc2(F.gelu(fc1(h))), pred, i == 0, 7)
+                delta = fc2(F.gelu(fc1(h))).float()
+                pred = delta if i == 0 else pred + delta
+                act, src = self.activate(pred), pred.half()
             outs.append(act)
         return outs
 

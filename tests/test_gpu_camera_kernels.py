@@ -141,3 +141,35 @@ def test_w4a16_ln_linear(gpu, M, N, K, gelu):
     ref = torch.nn.functional.gelu(lin) if gelu else lin
     term = (h.double().abs().mean() * 0.05)
     assert ((got - ref).abs() <= ref.abs() * 2.0 ** -10 + term * 2.0 ** -11 * K ** 0.5 + 1e-4).all()
+
+
+def _head_and_tokens(gpu, S=3):
+    from qvggt_amd.camera_head import CameraHead
+    return CameraHead.random(seed=2, device=gpu), torch.randn(
+        S, 2048, generator=torch.Generator(device=gpu).manual_seed(1), device=gpu).half()
+
+
+def _rel(a, b):
+    return max(((x - y).abs().max() / y.abs().max()).item() for x, y in zip(a, b))
+
+
+def test_camera_head_activation_can_be_replaced(gpu):
+    """``activate`` of a subclass or of an instance makes the outputs, and one
+    that returns its argument is not overwritten by the next iteration."""
+    from qvggt_amd.camera_head import CameraHead
+
+    class Plain(CameraHead):
+        @staticmethod
+        def activate(enc):
+            return enc
+
+    head, t = _head_and_tokens(gpu)
+    want = head(t)
+    head.__class__ = Plain
+    got = head(t)
+    assert any((o[:, 7:] < 0).any() for o in got) and _rel([CameraHead.activate(o) for o in got], want) <= 1e-2
+    head.__class__ = CameraHead
+    head.activate = lambda enc: 2 * CameraHead.activate(enc)
+    assert _rel([o / 2 for o in head(t)], want) <= 1e-2
+    del head.activate
+    assert all(torch.equal(a, b) for a, b in zip(head(t), want))
