@@ -61,25 +61,37 @@ POSE_ATTENTION_MAX = 256
 POSE_LINEAR_MAX = 64
 
 
-def _plain(*modules) -> bool:
-    """Whether calling the modules does nothing but their own forward: no hooks
-    on them or on all modules, the linears plain fp16 ones with a bias and
-    weights that 16-byte loads can read."""
+def _unhooked(*modules) -> bool:
+    """Whether calling the modules does nothing but their own forward."""
     g = nn.modules.module
     if g._global_forward_hooks or g._global_forward_pre_hooks or g._global_backward_hooks or g._global_backward_pre_hooks:
         return False
-    for m in modules:
-        if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__:
-            return False
-        if isinstance(m, nn.Linear):
-            p = m._parameters
-            if (type(m) is not nn.Linear or p.get("weight") is None or p.get("bias") is None
-                    or p["weight"].dtype != torch.float16 or p["bias"].dtype != torch.float16
-                    or p["weight"].data_ptr() % 16):
-                return False
-        elif type(m) not in (nn.Sequential, nn.SiLU):
-            return False
-    return True
+    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                   or "forward" in m.__dict__ for m in modules)
+
+
+def _plain_linear(m, k: int, n: int | None = None) -> bool:
+    """Whether m is a plain fp16 linear from k (to n) channels with a bias and
+    weights that 16-byte loads can read."""
+    if type(m) is not nn.Linear:
+        return False
+    w, b = m._parameters.get("weight"), m._parameters.get("bias")
+    return (type(w) is nn.Parameter and type(b) is nn.Parameter and w.dtype == b.dtype == torch.float16
+            and w.dim() == 2 and w.shape[1] == k and n in (None, w.shape[0]) and b.shape == w.shape[:1]
+            and w.data_ptr() % 16 == 0)
+
+
+def _fusable(embed, modulation, fc1, fc2) -> bool:
+    """Whether the head's own modules are what the few-token kernels compute:
+    embed, (SiLU, linear), fc1 and fc2 as built here, or of other inner widths
+    that the kernels' K steps of 32 divide."""
+    if type(modulation) is not nn.Sequential or len(modulation) != 2:
+        return False
+    silu, lin = modulation
+    return (type(silu) is nn.SiLU and _plain_linear(embed, POSE_DIM) and _plain_linear(lin, embed.weight.shape[0], 3 * DIM)
+            and _plain_linear(fc1, DIM) and _plain_linear(fc2, fc1.weight.shape[0], POSE_DIM)
+            and lin.weight.shape[1] % 32 == 0 and fc2.weight.shape[1] % 32 == 0
+            and _unhooked(embed, modulation, silu, lin, fc1, fc2))
 
 
 def _norm_linear(norm, layer, x: torch.Tensor, epilogue: int, n: int) -> torch.Tensor:
@@ -213,7 +225,7 @@ class CameraHead(nn.Module):
         outs = []
         embed, modulation, fc1, fc2 = self.embed_pose, self.poseLN_modulation, self.pose_branch.fc1, self.pose_branch.fc2
         kernel_act = self.activate is activate_pose
-        fused = (kernel_act and S <= POSE_LINEAR_MAX and _plain(embed, modulation, *modulation, fc1, fc2)
+        fused = (kernel_act and S <= POSE_LINEAR_MAX and _fusable(embed, modulation, fc1, fc2)
                  and not torch.is_autocast_enabled())
         for i in range(num_iterations):
             if fused:

@@ -143,10 +143,29 @@ def test_w4a16_ln_linear(gpu, M, N, K, gelu):
     assert ((got - ref).abs() <= ref.abs() * 2.0 ** -10 + term * 2.0 ** -11 * K ** 0.5 + 1e-4).all()
 
 
+class _Call(torch.nn.Module):
+    """A module that calls another: no longer one that the head can look into."""
+
+    def __init__(self, inner, post=lambda y: y):
+        super().__init__()
+        self.inner, self.post = inner, post
+
+    def forward(self, x):
+        return self.post(self.inner(x))
+
+
 def _head_and_tokens(gpu, S=3):
     from qvggt_amd.camera_head import CameraHead
     return CameraHead.random(seed=2, device=gpu), torch.randn(
         S, 2048, generator=torch.Generator(device=gpu).manual_seed(1), device=gpu).half()
+
+
+def _linear(gpu, k, n, seed):
+    l = torch.nn.Linear(k, n, device=gpu, dtype=torch.float16)
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    l.weight.data.copy_(torch.randn(n, k, generator=g, device=gpu) * 0.02)
+    l.bias.data.copy_(torch.randn(n, generator=g, device=gpu) * 0.02)
+    return l
 
 
 def _rel(a, b):
@@ -173,3 +192,26 @@ def test_camera_head_activation_can_be_replaced(gpu):
     assert _rel([o / 2 for o in head(t)], want) <= 1e-2
     del head.activate
     assert all(torch.equal(a, b) for a, b in zip(head(t), want))
+
+
+@pytest.mark.parametrize("kind", ["low_rank", "appended", "order", "narrow", "call"])
+def test_camera_head_modulation_can_be_replaced(gpu, kind):
+    """A ``poseLN_modulation`` of another build runs as built: equal, bit for
+    bit, to the same modules behind a module that the head cannot look into."""
+    from qvggt_amd.camera_head import _fusable
+    head, t = _head_and_tokens(gpu)
+    assert _fusable(head.embed_pose, head.poseLN_modulation, head.pose_branch.fc1, head.pose_branch.fc2)
+    silu, lin = head.poseLN_modulation
+    seq = {"low_rank": lambda: torch.nn.Sequential(silu, _linear(gpu, 2048, 64, 5), _linear(gpu, 64, 6144, 6)),
+           "appended": lambda: torch.nn.Sequential(silu, lin, torch.nn.SiLU()),
+           "order": lambda: torch.nn.Sequential(lin, torch.nn.SiLU()),
+           "narrow": lambda: torch.nn.Sequential(silu, _linear(gpu, 100, 6144, 7)),
+           "call": lambda: _Call(head.poseLN_modulation)}[kind]()
+    if kind == "narrow":
+        head.embed_pose = _linear(gpu, 9, 100, 8)
+    own = (head.embed_pose, head.pose_branch.fc1, head.pose_branch.fc2)
+    assert _fusable(own[0], seq, *own[1:]) is False
+    head.poseLN_modulation = seq
+    got = head(t)
+    head.poseLN_modulation = _Call(seq)
+    assert all(torch.equal(a, b) for a, b in zip(got, head(t)))
