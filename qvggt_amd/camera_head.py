@@ -94,6 +94,17 @@ def _fusable(embed, modulation, fc1, fc2) -> bool:
             and _unhooked(embed, modulation, silu, lin, fc1, fc2))
 
 
+def _modulate(mod: torch.Tensor, adaln: torch.Tensor, pose: torch.Tensor) -> torch.Tensor:
+    """gate * (adaln * (1 + scale) + shift) + pose for mod = (shift | scale | gate):
+    one kernel for the modulation that the head's own modules make, torch for
+    what else a replaced one returns (another type, one row for all frames)."""
+    S, D = pose.shape
+    if mod.dtype == pose.dtype == torch.float16 and mod.shape == (S, 3 * D) and _aligned(mod):
+        return E.adaln_modulate(mod, adaln, pose)
+    shift, scale, gate = mod.chunk(3, dim=-1)
+    return (gate * (adaln * (1 + scale) + shift) + pose).contiguous()
+
+
 def _norm_linear(norm, layer, x: torch.Tensor, epilogue: int, n: int) -> torch.Tensor:
     """layer(norm(x)) with its bias (+ GELU): one kernel for a ``WQLinear`` on up
     to 16 tokens (one MFMA tile; 6.3-9.0 us against 7.5-9.5 for the two, and
@@ -231,18 +242,19 @@ class CameraHead(nn.Module):
             if fused:
                 x = E.pose_modulate(E.pose_embed(src, *_affine(embed)), *_affine(modulation[1]), adaln, pose)
             else:
-                x = E.adaln_modulate(modulation(embed(src)), adaln, pose)
+                x = _modulate(modulation(embed(src)), adaln, pose)
             for blk in self.trunk:
                 blk(x)
             h = E.layer_norm(x, *_affine(self.trunk_norm), LN_EPS)
             if fused:
                 act, src = E.pose_delta(E.pose_linear_gelu(h, *_affine(fc1)), *_affine(fc2), pred, i == 0, POSE_LINEAR)
-            elif kernel_act:
-                act, src = E.pose_update(fc2(F.gelu(fc1(h))), pred, i == 0, POSE_LINEAR)
             else:
-                delta = fc2(F.gelu(fc1(h))).float()
-                pred = delta if i == 0 else pred + delta
-                act, src = self.activate(pred), pred.half()
+                delta = fc2(F.gelu(fc1(h)))
+                if kernel_act and delta.dtype == torch.float16 and delta.shape == pred.shape:
+                    act, src = E.pose_update(delta, pred, i == 0, POSE_LINEAR)
+                else:
+                    pred = delta.float() if i == 0 else pred + delta.float()
+                    act, src = self.activate(pred), pred.half()
             outs.append(act)
         return outs
 

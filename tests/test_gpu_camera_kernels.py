@@ -215,3 +215,31 @@ def test_camera_head_modulation_can_be_replaced(gpu, kind):
     got = head(t)
     head.poseLN_modulation = _Call(seq)
     assert all(torch.equal(a, b) for a, b in zip(got, head(t)))
+
+
+def test_camera_head_pose_branch_can_be_replaced(gpu):
+    """Pose branches of other widths, and one that ends in fp32."""
+    head, t = _head_and_tokens(gpu)
+    want = head(t)
+    fc1, fc2 = head.pose_branch.fc1, head.pose_branch.fc2
+    head.pose_branch.fc2 = _Call(fc2, lambda y: y.float())
+    assert _rel(head(t), want) <= 1e-2
+    head.pose_branch.fc1, head.pose_branch.fc2 = _linear(gpu, 2048, 100, 3), _linear(gpu, 100, 9, 4)
+    got = head(t)
+    head.pose_branch.fc2 = _Call(head.pose_branch.fc2)
+    assert _rel(got, head(t)) <= 1e-2
+
+
+@pytest.mark.parametrize("post", ["one_row", "unaligned"])
+def test_camera_head_takes_modulations_of_other_forms(gpu, post):
+    """One modulation row for all frames, and one off 16-byte addresses."""
+    head, t = _head_and_tokens(gpu)
+    mod = head.poseLN_modulation
+
+    def unaligned(y):
+        return torch.empty(y.numel() + 1, device=gpu, dtype=y.dtype)[1:].view_as(y).copy_(y)
+
+    head.poseLN_modulation = _Call(mod, (lambda y: y[:1]) if post == "one_row" else unaligned)
+    got = head(t)
+    head.poseLN_modulation = _Call(mod, (lambda y: y[:1].expand(3, -1)) if post == "one_row" else lambda y: y)
+    assert _rel(got, head(t)) <= 1e-2
