@@ -274,8 +274,21 @@ def _affine(ln: nn.Module):
 
 
 def _aligned(*tensors: torch.Tensor) -> bool:
-    """Whether the fp16 linear's 16-byte accesses may read and write them."""
+    """Whether 16-byte accesses may read and write them."""
     return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def _f16_fusable(x: torch.Tensor, weight, bias, out: torch.Tensor, gamma=None) -> bool:
+    """Whether ``f16_linear`` takes a linear of x (M, K) into out (with gamma,
+    its LayerScale update of out): fp16 throughout, one bias and one gamma a
+    channel, out whole, nothing off 16-byte addresses."""
+    M, K = x.shape
+    N = weight.shape[0]
+    f16 = torch.float16
+    return (weight.dtype == bias.dtype == out.dtype == f16 and weight.shape == (N, K) and bias.shape == (N,)
+            and out.shape == (M, N) and out.is_contiguous() and K % 32 == 0 and N % 16 == 0
+            and (gamma is None or (gamma.dtype == f16 and gamma.shape == (N,) and _aligned(gamma)))
+            and _aligned(x, weight, bias, out))
 
 
 def _with_depth(cfg: AggregatorConfig, depth: int | None) -> AggregatorConfig:
@@ -390,13 +403,13 @@ class DinoBlock(nn.Module):
         att = E.attention(*v3.unbind(1), TOKENS, out=ws["att"].view(M, HEADS, HEAD_DIM))
         proj_w, proj_b = _affine(attn.proj)
         gamma1 = self.ls1.gamma
-        if x.is_contiguous() and _aligned(x, att, proj_w, proj_b, gamma1):
+        if _f16_fusable(att.view(M, DIM), proj_w, proj_b, x, gamma1):
             E.f16_linear(att.view(M, DIM), proj_w, proj_b, out=x, gamma=gamma1)
         else:
             x.addcmul_(torch.addmm(proj_b, att.view(M, DIM), proj_w.t(), out=ws["o"]), gamma1)
         h = E.layer_norm(x, *_affine(self.norm2), self.eps, out=ws["h"])
         fc1_w, fc1_b = _affine(mlp.fc1)
-        if _aligned(h, fc1_w, fc1_b, ws["f"]):
+        if _f16_fusable(h, fc1_w, fc1_b, ws["f"]):
             f = E.f16_linear(h, fc1_w, fc1_b, QV_EPI_BIAS_GELU, out=ws["f"])
         else:
             f = F.gelu(torch.addmm(fc1_b, h, fc1_w.t(), out=ws["f"]))

@@ -226,3 +226,25 @@ def test_dino_block_takes_strided_and_unaligned_tensors(gpu):
     off = blk(x.clone(), ws)
     for y in (got, off):
         assert (y.float() - want.float()).abs().max().item() <= 2.0 ** -9 * want.float().abs().max().item()
+
+
+@pytest.mark.parametrize("gamma", ["float32", "one"])
+def test_dino_block_takes_any_layer_scale(gpu, gamma):
+    """An fp32 LayerScale, or one of a single element, as torch's addcmul takes
+    them: within two fp16 steps of the fp16 vector of the same values."""
+    from qvggt_amd import aggregator as AG
+    agg = AG.Aggregator.random(seed=6, device=gpu, depth=1)
+    blk, M = agg.patch_embed.blocks[0], AG.TOKENS
+    ws = agg._workspace(M, gpu)
+    blk.ls1.gamma.fill_(0.5)
+    blk.ls2.gamma.fill_(0.5)
+    x = torch.randn(M, AG.DIM, generator=torch.Generator(device=gpu).manual_seed(2), device=gpu).half()
+    proj = blk.attn.proj
+    assert AG._f16_fusable(ws["att"], proj.weight, proj.bias, x, blk.ls1.gamma)
+    assert AG._f16_fusable(ws["h"], blk.mlp.fc1.weight, blk.mlp.fc1.bias, ws["f"])
+    want = blk(x.clone(), ws)
+    g = torch.full((AG.DIM,), 0.5, device=gpu) if gamma == "float32" else torch.full((1,), 0.5, device=gpu).half()
+    blk.ls1.gamma = torch.nn.Parameter(g, requires_grad=False)
+    assert not AG._f16_fusable(ws["att"], proj.weight, proj.bias, x, blk.ls1.gamma)
+    got = blk(x.clone(), ws)
+    assert (got.float() - want.float()).abs().max().item() <= 2.0 ** -9 * want.float().abs().max().item()
