@@ -631,7 +631,7 @@ extern "C" int qv_f16_gemm(const void* x, const void* w, const void* bias, const
   QV_CHECK_ARG(M >= 0 && N > 0 && K > 0, "bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
   QV_CHECK_ARG(K % 32 == 0 && N % 16 == 0, "K=%lld must be a multiple of 32 and N=%lld of 16", (long long)K, (long long)N);
   QV_CHECK_ARG(M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX / 2, "shape too large");
-  QV_CHECK_ARG((uint64_t)N * K * 2 < (1ull << 32) && (uint64_t)256 * K < (1ull << 31),
+  QV_CHECK_ARG((uint64_t)N * K * 2 < (1ull << 32) && (uint64_t)256 * K * 2 < (1ull << 31),
                "weight too large for 32-bit offsets");
   QV_CHECK_ARG(epilogue == QV_EPI_BIAS || epilogue == QV_EPI_BIAS_GELU, "unsupported epilogue %d", epilogue);
   QV_CHECK_ARG(!gamma || epilogue == QV_EPI_BIAS, "the residual form takes the bias epilogue");

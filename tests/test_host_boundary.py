@@ -222,6 +222,19 @@ def test_w4a16_plan_rules(M, N, K, epi, kind, tile, tile2):
         assert 0 < p["rows"] <= M and (p["tile2"] or p["rows"] == M)
 
 
+def test_f16_gemm_refuses_rows_past_32_bit_offsets():
+    """The kernel's row offsets inside a tile (up to 255 rows of 2 K bytes) are
+    32-bit signed: K = 2^22 would overflow them, the next smaller multiple of
+    32 does not.  M = 0, so nothing is launched."""
+    for k, ok in ((2 ** 22 - 32, True), (2 ** 22, False), (2 ** 23 - 32, False)):
+        args = (None, None, None, None, None, 0, 16, k, 1, None)
+        if ok:
+            _lib.call("qv_f16_gemm", *args)
+        else:
+            with pytest.raises(RuntimeError, match="32-bit offsets"):
+                _lib.call("qv_f16_gemm", *args)
+
+
 def test_w4a16_plan_rejects_bad_shapes():
     for args in [(0, 64, 128, 0), (8, 64, 100, 0), (8, 60, 128, 0), (8, 64, 128, 9)]:
         with pytest.raises(RuntimeError):
