@@ -322,6 +322,15 @@ int qv_attention_fwd(const void* q, const void* k, const void* v, void* out, int
                      int64_t k_token_stride, int64_t v_token_stride, int64_t out_token_stride,
                      float scale, void* stream);
 
+/*
+ * The launch form that an int8 GEMM (kind 0: weight as stored, 1: packed, 2:
+ * int32 output) or qv_f16_gemm (kind 3) picks for M x K -> N, written to
+ * plan[2]: plan[0] = rows of a tile (32, 64, 96 or 128), plan[1] = 2 if K is
+ * split between two wave groups of one workgroup, else 1.  No device work; for
+ * tests and profiling.
+ */
+int qv_w8a8_plan(int64_t M, int64_t N, int64_t K, int kind, int32_t* plan);
+
 /* ---------------------------------------------------- fp16 linear
  * No counterpart in the reference extension (the DINOv2 patch embed stays in
  * floating point, qvggt/inference/loader.py:346, and its graph is in the

@@ -53,6 +53,7 @@ SIGNATURES: dict[str, list] = {
     "qv_rope2d": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp],
     "qv_qknorm_rope2d": [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _f32, _i64, _i64, _i64, _vp],
     "qv_w4a16_ln_linear": [_vp, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
+    "qv_w8a8_plan": [_i64, _i64, _i64, _i32, _vp],
     "qv_f16_gemm": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i32, _vp],
     "qv_pose_attention": [_vp, _vp, _i64, _i64, _i64, _f32, _vp],
     "qv_pose_embed": [_vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _vp],

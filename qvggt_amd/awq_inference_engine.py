@@ -501,6 +501,15 @@ def w8a8_linear_residual(in_feats, kernel, wscales, ascales, bias, gamma, residu
     return residual
 
 
+def w8a8_plan(M: int, N: int, K: int, kind: str = "stored") -> tuple:
+    """(tile rows, K split) of the launch form that an int8 GEMM ("stored",
+    "packed" or "int32") or ``f16_linear`` ("fp16") picks; no device work."""
+    plan = (C.c_int32 * 2)()
+    _lib.call("qv_w8a8_plan", int(M), int(N), int(K), ("stored", "packed", "int32", "fp16").index(kind),
+              C.cast(plan, C.c_void_p))
+    return plan[0], plan[1]
+
+
 def w8a8_packed_bytes(N: int, K: int) -> int:
     """Size in bytes of an (N, K) int8 weight in the packed layout (N rounded up to 32)."""
     return (N + 31) // 32 * 32 * K

@@ -654,6 +654,18 @@ extern "C" int qv_f16_gemm(const void* x, const void* w, const void* bias, const
   return check_launch("f16_gemm");
 }
 
+extern "C" int qv_w8a8_plan(int64_t M, int64_t N, int64_t K, int kind, int32_t* plan) {
+  QV_CHECK_ARG(plan != nullptr, "null plan pointer");
+  QV_CHECK_ARG(kind >= 0 && kind <= 3, "bad kind %d", kind);
+  QV_CHECK_ARG(M > 0 && N > 0 && K > 0 && K % (kind == 3 ? 32 : 64) == 0 && N % 16 == 0 && M <= INT32_MAX &&
+                   N <= INT32_MAX && K <= INT32_MAX / 2,
+               "bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
+  const int form = qv::w8a8_form(M, N, kind == 3 ? 2 * K : K, kind == 1, kind <= 1);
+  plan[0] = 32 * (form / 10);
+  plan[1] = form % 10;
+  return QV_OK;
+}
+
 extern "C" int qv_w8a8_gemm(const int8_t* a, const int8_t* b, const void* wscales, const void* ascales,
                             const void* bias, void* out, int64_t M, int64_t N, int64_t K, void* stream) {
   return qv::w8a8_run(a, b, wscales, ascales, bias, nullptr, out, M, N, K, bias ? 1 : 0, stream);

@@ -547,15 +547,25 @@ def test_qknorm_rope2d_bit_exact(gpu, H, S):
     assert np.array_equal(got[:, 2], x[:, 2])
 
 
-@pytest.mark.parametrize("M,N,K", [(500, 1024, 1024), (33, 272, 192), (65, 1024, 4096), (1373, 4096, 1024), (97, 272, 4096),
-                                   (4122, 1024, 4096), (4037, 1040, 2176), (1374, 1024, 4096), (64, 16, 2304),
-                                   (2000, 1024, 2112), (5496, 3072, 1024)])
-def test_w8a8_launch_forms_bit_exact(gpu, M, N, K):
+# (M, N, K), the (tile rows, K split) of its launch on the stored and on the packed layout
+W8_FORMS = [((500, 1024, 1024), (32, 1), (32, 1)), ((33, 272, 192), (32, 1), (32, 1)), ((65, 1024, 4096), (32, 1), (32, 1)),
+            ((1373, 4096, 1024), (96, 1), (96, 1)), ((97, 272, 4096), (32, 1), (32, 1)), ((4122, 1024, 4096), (96, 2), (96, 2)),
+            ((4037, 1040, 2176), (96, 2), (96, 2)), ((1374, 1024, 4096), (64, 2), (64, 2)), ((64, 16, 2304), (32, 1), (32, 1)),
+            ((2000, 1024, 2112), (64, 1), (64, 1)), ((5496, 3072, 1024), (96, 1), (96, 1)), ((9001, 272, 192), (96, 1), (64, 1)),
+            ((9001, 272, 2048), (96, 2), (96, 2)), ((2049, 272, 2048), (64, 2), (64, 2)), ((2049, 272, 2176), (64, 2), (64, 2)),
+            ((5501, 2064, 192), (128, 1), (128, 1)), ((10992, 4096, 1024), (128, 1), (128, 1))]
+
+
+@pytest.mark.parametrize("shape,stored,packed", W8_FORMS)
+def test_w8a8_launch_forms_bit_exact(gpu, shape, stored, packed):
     """The launch forms (32-, 64-, 96-, 128-row tiles; K split between two wave
     groups, odd and even stage counts a group, K that cannot be split) on both
-    weight layouts and the residual form: the integer sums are exact (float64
-    products), so every form gives the epilogue's bits."""
+    weight layouts, without bias, with it and in the residual form: the integer
+    sums are exact (float64 products), so every form gives the epilogue's bits.
+    The plan says that each shape runs the form that it is here for."""
     from qvggt_amd import awq_inference_engine as E
+    M, N, K = shape
+    assert E.w8a8_plan(M, N, K) == stored and E.w8a8_plan(M, N, K, "packed") == packed
     g = torch.Generator(device=gpu).manual_seed(M + N + K)
     a, w = (torch.randint(-128, 128, sh, generator=g, device=gpu, dtype=torch.int16).to(torch.int8) for sh in ((M, K), (N, K)))
     ws, as_ = (torch.rand(n, generator=g, device=gpu).mul(1e-3).half() for n in (N, M))
@@ -564,13 +574,18 @@ def test_w8a8_launch_forms_bit_exact(gpu, M, N, K):
     acc = (a.double() @ w.double().t().contiguous()).float()
     want = (acc * ws.float()[None] * as_.float()[:, None] + bias.float()[None]).half()
     want_res = (res.float() + gamma.float()[None] * want.float()).half()
-    packed = E.w8a8_pack_weight(w)
-    out = [torch.full((M, N), float("nan"), device=gpu, dtype=torch.float16) for _ in range(2)]
+    want_plain = (acc * ws.float()[None] * as_.float()[:, None]).half()
+    pw = E.w8a8_pack_weight(w)
+    plain, out = ([torch.full((M, N), float("nan"), device=gpu, dtype=torch.float16) for _ in range(2)] for _ in range(2))
+    E.w8a8_gemm_forward_cuda(a, w, ws, as_, plain[0])
+    E.w8a8_gemm_packed(a, pw, N, ws, as_, plain[1])
     E.w8a8_gemm_fuse_bias_forward_cuda(a, w, ws, as_, out[0], bias)
-    E.w8a8_gemm_packed(a, packed, N, ws, as_, out[1], bias=bias)
+    E.w8a8_gemm_packed(a, pw, N, ws, as_, out[1], bias=bias)
     r = [res.clone(), res.clone()]
     E.w8a8_linear_residual(a, w, ws, as_, bias, gamma, r[0])
-    E.w8a8_gemm_packed(a, packed, N, ws, as_, r[1], bias=bias, gamma=gamma)
+    E.w8a8_gemm_packed(a, pw, N, ws, as_, r[1], bias=bias, gamma=gamma)
+    for o in plain:
+        assert torch.equal(o, want_plain)
     for o in out:
         assert torch.equal(o, want)
     for o in r:
@@ -578,16 +593,19 @@ def test_w8a8_launch_forms_bit_exact(gpu, M, N, K):
     assert torch.equal(E.w8a8_gemm_int32(a, w).float(), acc)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (33, 272, 96), (65, 1024, 1024), (97, 1040, 160), (1374, 4096, 1024),
-                                   (4122, 1024, 1024), (5497, 4096, 1024)])
+@pytest.mark.parametrize("M,N,K,rows", [(1, 16, 32, 32), (33, 272, 96, 32), (65, 1024, 1024, 32), (97, 1040, 160, 32),
+                                        (1374, 1024, 1024, 64), (2749, 272, 160, 64), (1374, 4096, 1024, 96),
+                                        (4122, 1024, 1024, 96), (9001, 272, 96, 96), (5497, 4096, 1024, 128),
+                                        (2749, 2064, 160, 128)])
 @pytest.mark.parametrize("mode", ["bias", "gelu", "residual"])
-def test_f16_linear(gpu, M, N, K, mode):
-    """fp16 linear on the int8 kernel's pipeline, all tile heights and their
-    remainders, one to sixteen times two stages, against float64.  Bounds: one
+def test_f16_linear(gpu, M, N, K, rows, mode):
+    """fp16 linear on the int8 kernel's pipeline, all tile heights (the plan
+    says which) and their remainders, one to thirty-two stages, against float64.  Bounds: one
     fp16 rounding (2^-11 relative; the residual form rounds the linear and the
     sum; GELU's polynomial is within one more step, 2^-10), plus the fp32 sum's
     K * 2^-24 of the absolute terms."""
     from qvggt_amd import awq_inference_engine as E
+    assert E.w8a8_plan(M, N, K, "fp16") == (rows, 1)
     g = torch.Generator(device=gpu).manual_seed(M + N + K)
     x, w, b, ga, r = (torch.randn(sh, generator=g, device=gpu).mul(sc).half() for sh, sc in
                       (((M, K), 1.0), ((N, K), K ** -0.5), ((N,), 0.5), ((N,), 0.5), ((M, N), 1.0)))

@@ -235,6 +235,26 @@ def test_f16_gemm_refuses_rows_past_32_bit_offsets():
                 _lib.call("qv_f16_gemm", *args)
 
 
+def test_w8a8_plan():
+    """The int8 and fp16 GEMMs' launch forms (host-side choice): only the fp16
+    outputs of the int8 GEMM split K, in 64- and 96-row tiles and only where K
+    gives both wave groups whole stages; bad shapes are refused."""
+    seen = {kind: set() for kind in ("stored", "packed", "int32", "fp16")}
+    for kind, forms in seen.items():
+        for K in (192, 1024, 2048, 2112, 4096):
+            for N in (272, 1024, 4096):
+                for M in (1, 97, 500, 1374, 2049, 4122, 5501, 10992):
+                    rows, ksplit = E.w8a8_plan(M, N, K, kind)
+                    assert ksplit == 1 or (kind in ("stored", "packed") and K >= 2048 and K % 128 == 0)
+                    forms.add((rows, ksplit))
+    one = {(32, 1), (64, 1), (96, 1), (128, 1)}
+    assert seen["int32"] == seen["fp16"] == one
+    assert seen["stored"] == seen["packed"] == one | {(64, 2), (96, 2)}
+    for bad in ((0, 64, 64), (8, 60, 64), (8, 64, 96), (8, 64, 0)):
+        with pytest.raises(RuntimeError):
+            E.w8a8_plan(*bad)
+
+
 def test_w4a16_plan_rejects_bad_shapes():
     for args in [(0, 64, 128, 0), (8, 64, 100, 0), (8, 60, 128, 0), (8, 64, 128, 9)]:
         with pytest.raises(RuntimeError):
