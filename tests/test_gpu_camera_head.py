@@ -36,6 +36,25 @@ def test_camera_head_w4_matches_oracle(gpu, S):
         assert got.shape == (S, 9) and np.isfinite(got).all() and err <= 1e-2, (i, err)
 
 
+@pytest.mark.parametrize("S", [64, 65, 256, 257])
+def test_camera_head_on_both_sides_of_its_switches(gpu, S):
+    """The last frame count of the fused linears and the first of the module
+    path, the last of the pose attention kernel and the first of torch's
+    products; two iterations, so that the pose update adds.  An fp16 trunk: the
+    switches are its callers', and the oracle needs no dequantisation."""
+    from qvggt_amd import camera_head as CH
+    assert {64, 256} == {CH.POSE_LINEAR_MAX, CH.POSE_ATTENTION_MAX}
+    head = CH.CameraHead.random(seed=S, device=gpu, w4=False)
+    t = np.random.default_rng(S).standard_normal((S, OC.DIM)).astype(np.float16)
+    outs = head(torch.from_numpy(t).to(gpu), num_iterations=2)
+    torch.cuda.synchronize()
+    ref = OC.camera_head(t.astype(np.float64), _params(head), num_iterations=2)
+    for i, (o, r) in enumerate(zip(outs, ref)):
+        got = o.cpu().numpy()
+        err = np.abs(got - r).max() / np.abs(r).max()
+        assert got.shape == (S, 9) and np.isfinite(got).all() and err <= 1e-2, (i, err)
+
+
 def test_camera_head_takes_camera_tokens_of_the_aggregator_output(gpu):
     """The head reads the camera token (token 0) of each frame of the last
     [frame | global] aggregator layer; frames stay independent of their order."""
