@@ -70,15 +70,18 @@ def _unhooked(*modules) -> bool:
                    or "forward" in m.__dict__ for m in modules)
 
 
-def _plain_linear(m, k: int, n: int | None = None) -> bool:
-    """Whether m is a plain fp16 linear from k (to n) channels with a bias and
-    weights that 16-byte loads can read."""
+def _plain_linear(m, k: int, n: int | None = None) -> int:
+    """The output channels of m if it is a plain fp16 linear from k (to n)
+    channels with a bias and weights that 16-byte loads can read, else 0."""
     if type(m) is not nn.Linear:
-        return False
+        return 0
     w, b = m._parameters.get("weight"), m._parameters.get("bias")
-    return (type(w) is nn.Parameter and type(b) is nn.Parameter and w.dtype == b.dtype == torch.float16
-            and w.dim() == 2 and w.shape[1] == k and n in (None, w.shape[0]) and b.shape == w.shape[:1]
-            and w.data_ptr() % 16 == 0)
+    if type(w) is not nn.Parameter or type(b) is not nn.Parameter:
+        return 0
+    shape = w.shape
+    ok = (w.dtype == b.dtype == torch.float16 and len(shape) == 2 and shape[1] == k and n in (None, shape[0])
+          and b.shape == shape[:1] and w.data_ptr() % 16 == 0)
+    return shape[0] if ok else 0
 
 
 def _fusable(embed, modulation, fc1, fc2) -> bool:
@@ -88,9 +91,9 @@ def _fusable(embed, modulation, fc1, fc2) -> bool:
     if type(modulation) is not nn.Sequential or len(modulation) != 2:
         return False
     silu, lin = modulation
-    return (type(silu) is nn.SiLU and _plain_linear(embed, POSE_DIM) and _plain_linear(lin, embed.weight.shape[0], 3 * DIM)
-            and _plain_linear(fc1, DIM) and _plain_linear(fc2, fc1.weight.shape[0], POSE_DIM)
-            and lin.weight.shape[1] % 32 == 0 and fc2.weight.shape[1] % 32 == 0
+    e, m = _plain_linear(embed, POSE_DIM), _plain_linear(fc1, DIM)
+    return (type(silu) is nn.SiLU and e > 0 and e % 32 == 0 and m > 0 and m % 32 == 0
+            and _plain_linear(lin, e, 3 * DIM) > 0 and _plain_linear(fc2, m, POSE_DIM) > 0
             and _unhooked(embed, modulation, silu, lin, fc1, fc2))
 
 
