@@ -337,7 +337,7 @@ int qv_w8a8_plan(int64_t M, int64_t N, int64_t K, int kind, int32_t* plan);
  * external vggt-hf): out = epilogue(x w^T + bias), x (M, K), w (N, K), bias (N)
  * fp16, fp32 sums, one rounding.  epilogue QV_EPI_BIAS or QV_EPI_BIAS_GELU;
  * with gamma (N, QV_EPI_BIAS only) out += gamma * fp16(x w^T + bias) in place.
- * K a multiple of 32, N of 16; x, w, out and gamma 16-byte, bias 8-byte aligned.
+ * K a multiple of 32 below 2^22, N of 16; x, w, out and gamma 16-byte, bias 8-byte aligned.
  */
 int qv_f16_gemm(const void* x, const void* w, const void* bias, const void* gamma, void* out,
                 int64_t M, int64_t N, int64_t K, int epilogue, void* stream);

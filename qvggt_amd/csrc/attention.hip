@@ -368,7 +368,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(QB =
       issue_k(j + 1, buf ^ 1);
       issue_v(j + 1, buf ^ 1);
     }
-    // a wave whose 64 queries all lie past the sequence end (the last query
+    // a wave whose queries all lie past the sequence end (the last query
     // tile of a frame) only issues its share of the DMA and keeps the barriers
     if (live) {
 #pragma unroll

@@ -6,7 +6,9 @@
 // by its launch and by one or two memory latencies, not by bytes or
 // arithmetic; what pays is doing in one launch what the chain did in several.
 // As torch ops the attention took 9 launches, the modulation 7, the pose update
-// 5: the eager head at 8 frames went from 4.0 to 2.3 ms, ~400 launches to ~150.
+// 5: the eager head at 8 frames went from 4.0 to 2.3 ms; with its own linears
+// here too (below) and the trunk's norms in their linears, to 1.15 ms and from
+// ~400 launches to 102.
 #include <type_traits>
 
 #include "common.h"

@@ -545,7 +545,10 @@ static void launch(const void* a, const void* b, const void* ws, const void* as,
 // past half the chip only for short K on the packed layout (1374 x 4096 ->
 // 1024: 18.5 us packed and 33.3 stored, against 15.6 and 22.3 for 64 rows, K
 // split).  128 rows with K split spill; 32 rows with K split were nowhere better by
-// more than 4 %.
+// more than 4 %.  On 84 launches it was not fitted to (the same layers, 70-12288
+// rows): 1.0 / 1.2 % off the best (stored / packed), 5 / 10 % faster than the
+// former rule, at worst 3 % slower (stored, 11500-12288 x 4096 -> 1024).  On other
+// layers (K 512-6144, N 768-6144) 1.2 / 3.1 % off, 5 / 7 % faster.
 static int w8a8_form(int64_t M, int64_t N, int64_t K, bool packed, bool ksplit) {
   struct Form { int form; float s0, s1, p0, p1; };
   static const Form forms[2][6] = {
@@ -623,8 +626,13 @@ static int w8a8_run(const void* a, const void* b, const void* ws, const void* as
 // a clock at full MFMA rate against 128.  What it gains over the library's
 // product is the fused epilogue: bias + GELU 1024 -> 4096 in 65.6 us against
 // 81 at M = 5496 (22.9 / 28.4 at 1374, 99.9 / 114 at 8244, 222 / 262 at 21984),
-// bias + residual 1024 -> 1024 in 25.2 against 18.5 + 9.5.  Without one (qkv),
-// or at K = 4096, the library's product is faster (43 / 52 us, 49 / 77).
+// bias + residual 1024 -> 1024 in 24.4 against 25.5 (13.4 / 22.2 at 1374, 28.8 /
+// 31.5 at 8244).  The estimate's constants are the int8 ones: over 84 launches
+// of these layers (70-12288 rows) the form is 1.6 % off the best; where it
+// errs most, K = 4096 from 10000 rows on (96-row tiles for 128, 4-10 %), the
+// library's product is the one to take.  Without an epilogue to fuse (qkv),
+// or at K = 4096, the library's product is faster (44 / 50 us; fc2 with its
+// residual update 54.5 / 75.8).
 extern "C" int qv_f16_gemm(const void* x, const void* w, const void* bias, const void* gamma, void* out, int64_t M,
                            int64_t N, int64_t K, int epilogue, void* stream) {
   using namespace qv;

@@ -59,11 +59,10 @@ def test_global_attention_s32_sampled_rows(gpu):
 
 
 def test_attention_two_forms_agree_bitwise(gpu):
-    """Launches that would not fill one round of 4-wave workgroups run the
-    2-wave form (64-key DMA tiles); every query sees its keys in the same
-    order in both forms, so the first 4 frames of an 8-frame launch (4-wave
-    form) equal a 4-frame launch on the same tokens (2-wave form) bit for bit,
-    and both meet the oracle."""
+    """A launch of 4 frames runs 32 queries a wave (64-key DMA tiles), one of 8
+    frames 64 queries a wave; every query sees its keys in the same order in
+    both forms, so the first 4 frames of the 8-frame launch equal the 4-frame
+    launch on the same tokens bit for bit, and both meet the oracle."""
     from qvggt_amd import awq_inference_engine as E
     L, H = 1374, 16
     x = _qkv(8 * L, H, 11)

@@ -82,9 +82,9 @@ def test_pose_linears(gpu, S, N, K):
     b, (a, p) = torch.randn(3 * N, generator=g, device=gpu).half(), torch.randn(2, S, N, generator=g, device=gpu).half()
     lin = x.double() @ w.double().t().contiguous() + b.double()
     _close(E.pose_modulate(x, w, b, a, p), lin[:, 2 * N:] * (a.double() * (1 + lin[:, N:2 * N]) + lin[:, :N]) + p.double(), 20.0)
-    # gelu: the polynomial is within one fp16 step more
+    # gelu: its fitted tail adds 3e-6 of the result
     got, ref = E.pose_linear_gelu(x, w[:N], b[:N]).double(), torch.nn.functional.gelu(lin[:, :N])
-    assert ((got - ref).abs() <= ref.abs() * (2.0 ** -11 + 2.0 ** -10) + 1e-4).all()
+    assert ((got - ref).abs() <= ref.abs() * (2.0 ** -11 + 4e-6) + 1e-4).all()
     pred = torch.randn(S, 9, generator=g, device=gpu)
     want = pred.double() + lin[:, :9]
     act, half = E.pose_delta(x, w[:9], b[:9], pred, False, 7)

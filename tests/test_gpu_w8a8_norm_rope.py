@@ -600,10 +600,10 @@ def test_w8a8_launch_forms_bit_exact(gpu, shape, stored, packed):
 @pytest.mark.parametrize("mode", ["bias", "gelu", "residual"])
 def test_f16_linear(gpu, M, N, K, rows, mode):
     """fp16 linear on the int8 kernel's pipeline, all tile heights (the plan
-    says which) and their remainders, one to thirty-two stages, against float64.  Bounds: one
-    fp16 rounding (2^-11 relative; the residual form rounds the linear and the
-    sum; GELU's polynomial is within one more step, 2^-10), plus the fp32 sum's
-    K * 2^-24 of the absolute terms."""
+    says which) and their remainders, one to thirty-two stages, against
+    float64.  Bounds: one fp16 rounding (2^-11 relative; the residual form
+    rounds the linear and the sum; GELU's fitted tail adds 3e-6), plus the fp32
+    sum's K * 2^-24 of the absolute terms."""
     from qvggt_amd import awq_inference_engine as E
     assert E.w8a8_plan(M, N, K, "fp16") == (rows, 1)
     g = torch.Generator(device=gpu).manual_seed(M + N + K)
@@ -617,7 +617,7 @@ def test_f16_linear(gpu, M, N, K, rows, mode):
         bound = ref.abs() * 2.0 ** -11 + ga.double().abs() * (lin.abs() * 2.0 ** -11 + terms)
     elif mode == "gelu":
         got, ref = E.f16_linear(x, w, b, 2), torch.nn.functional.gelu(lin)
-        bound = ref.abs() * (2.0 ** -11 + 2.0 ** -10) + terms * 1.2
+        bound = ref.abs() * (2.0 ** -11 + 4e-6) + terms * 1.2
     else:
         got, ref, bound = E.f16_linear(x, w, b), lin, lin.abs() * 2.0 ** -11 + terms
     assert ((got.double() - ref).abs() <= bound + 2.0 ** -24).all()
